@@ -396,17 +396,12 @@ __global__ __launch_bounds__(KS_BLOCK) void k_ilu0_init(const int32_t *__restric
     for (int32_t q = rowptr[i]; q < rowptr[i + 1]; q++) lu[q] = val[q] - (colidx[q] == i ? sigma : 0.0);
 }
 
-// one level of the IKJ factorization (Saad, Algorithm 10.4): a thread per row of
-// the level; the rows it reads (its L part) belong to earlier levels.  The
-// operations of a row are the oracle's, in the same order.
-__global__ __launch_bounds__(64) void k_ilu0_factor_level(const int32_t *__restrict__ rows, int cnt,
-                                                         const int32_t *__restrict__ rowptr,
-                                                         const int32_t *__restrict__ colidx,
-                                                         const int32_t *__restrict__ diag, double *__restrict__ lu,
-                                                         int *zero_pivot) {
-  const int t = blockIdx.x * 64 + threadIdx.x;
-  if (t >= cnt) return;
-  const int i = rows[t];
+// row i of the IKJ factorization (Saad, Algorithm 10.4); the rows it reads (its
+// L part) belong to earlier levels.  The operations of a row are the oracle's,
+// in the same order.
+__device__ __forceinline__ void ilu0_factor_row(int i, const int32_t *__restrict__ rowptr,
+                                               const int32_t *__restrict__ colidx, const int32_t *__restrict__ diag,
+                                               double *lu, int *zero_pivot) {
   const int32_t re = rowptr[i + 1];
   for (int32_t q = rowptr[i]; q < diag[i]; q++) {
     const int k = colidx[q];
@@ -424,6 +419,34 @@ __global__ __launch_bounds__(64) void k_ilu0_factor_level(const int32_t *__restr
       while (u < ke && colidx[u] < j) u++;
       if (u < ke && colidx[u] == j) lu[r] -= lik * lu[u];
     }
+  }
+}
+
+// one level: a thread per row of the level
+__global__ __launch_bounds__(64) void k_ilu0_factor_level(const int32_t *__restrict__ rows, int cnt,
+                                                         const int32_t *__restrict__ rowptr,
+                                                         const int32_t *__restrict__ colidx,
+                                                         const int32_t *__restrict__ diag, double *__restrict__ lu,
+                                                         int *zero_pivot) {
+  const int t = blockIdx.x * 64 + threadIdx.x;
+  if (t < cnt) ilu0_factor_row(rows[t], rowptr, colidx, diag, lu, zero_pivot);
+}
+
+// every level in one workgroup, a barrier (which orders its global stores)
+// between them: for levels of at most KS_ILU_WG rows a launch a level costs
+// more than the level (128 x 127 grid, 254 levels: the whole set-up takes 3.1 ms
+// with a launch a level, 1.9 ms with one launch)
+#define KS_ILU_WG 1024
+__global__ __launch_bounds__(KS_ILU_WG) void k_ilu0_factor(const int32_t *__restrict__ rows,
+                                                          const int32_t *__restrict__ lptr, int nlev,
+                                                          const int32_t *__restrict__ rowptr,
+                                                          const int32_t *__restrict__ colidx,
+                                                          const int32_t *__restrict__ diag, double *lu,
+                                                          int *zero_pivot) {
+  for (int l = 0; l < nlev; l++) {
+    const int r = lptr[l] + (int)threadIdx.x;
+    if (r < lptr[l + 1]) ilu0_factor_row(rows[r], rowptr, colidx, diag, lu, zero_pivot);
+    __syncthreads();
   }
 }
 
@@ -491,6 +514,88 @@ __global__ __launch_bounds__(KS_BLOCK) void k_ilu0_sf(int n, const int32_t *__re
   }
 }
 
+// The same solve by one workgroup, one barrier a level, for dependency graphs
+// that are deep and narrow (a grid in natural order).  k_ilu0_sf hands a value
+// from row to row through memory, about 1.3 us a level whatever the level's
+// width; here the solved values stay in a ring in LDS and a level costs an LDS
+// round trip and a barrier.  Rows are laid out in level order, NT to a step and
+// each level padded to whole steps (row -1), their entries in E columns of a
+// fixed width (absent: coefficient 0 on the ring's zero slot), so every load is
+// coalesced and its address known in advance: KS_ILU_PD steps are in flight in
+// registers and the barrier waits for LDS only.  A row's subtractions keep
+// k_ilu0_sf's order, so the results are its bits.
+// 128 x 127 five-point grid (254 levels): one application of both factors 673
+// us by k_ilu0_sf, 114 us by levels (0.22 us a level).
+#define KS_ILU_PD 8
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+template <bool LOWER, int E, int NT>
+__global__ __launch_bounds__(NT) void k_ilu0_levels(int nsteps, int ring, const int32_t *__restrict__ rowid,
+                                                   const int32_t *__restrict__ dep, const double *__restrict__ coef,
+                                                   const double *__restrict__ dg, double *y, const ksp_state *S,
+                                                   int skip_sconv) {
+  if (S && (S->reason || (skip_sconv && S->sconv))) return;
+  extern __shared__ double xs[];   // ring values, then the zero slot
+  const int t = threadIdx.x;
+  const int np = nsteps * NT;      // at most a few times n: below 2^31
+  if (t == 0) xs[ring] = 0.0;
+  int rnext[KS_ILU_PD], r[KS_ILU_PD], d[KS_ILU_PD][E];
+  double c[KS_ILU_PD][E], b[KS_ILU_PD], g[KS_ILU_PD];
+  auto at = [&](int s) { return min(s, nsteps - 1) * NT + t; };
+  auto load = [&](int j, int s) {   // step s into slot j; its rows were loaded KS_ILU_PD steps before
+    const int p = at(s);
+    r[j] = rnext[j];
+    b[j] = y[max(r[j], 0)];
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+      d[j][e] = dep[e * np + p];
+      c[j][e] = coef[e * np + p];
+    }
+    if (!LOWER) g[j] = dg[p];
+    rnext[j] = rowid[at(s + KS_ILU_PD)];
+  };
+#pragma unroll
+  for (int j = 0; j < KS_ILU_PD; j++) rnext[j] = rowid[at(j)];
+#pragma unroll
+  for (int j = 0; j < KS_ILU_PD; j++) load(j, j);
+  lds_barrier();
+  for (int s0 = 0; s0 < nsteps; s0 += KS_ILU_PD) {
+#pragma unroll
+    for (int j = 0; j < KS_ILU_PD; j++) {
+      const int s = s0 + j;
+      if (s >= nsteps) break;
+      double v[E], x = b[j];
+#pragma unroll
+      for (int e = 0; e < E; e++) v[e] = xs[d[j][e]];
+#pragma unroll
+      for (int e = 0; e < E; e++) x -= c[j][e] * v[e];
+      if (!LOWER) x /= g[j];
+      xs[(s * NT + t) & (ring - 1)] = x;
+      if (r[j] >= 0) y[r[j]] = x;
+      load(j, s + KS_ILU_PD);
+      lds_barrier();
+    }
+  }
+}
+
+// coef[e][p] = the factor entry behind slot (e, p), dg[p] = its row's pivot
+__global__ __launch_bounds__(KS_BLOCK) void k_ilu0_pack(int np, int E, const int32_t *__restrict__ src,
+                                                       const int32_t *__restrict__ rowid,
+                                                       const int32_t *__restrict__ diag,
+                                                       const double *__restrict__ lu, double *__restrict__ coef,
+                                                       double *__restrict__ dg) {
+  KS_FOR_ROWS(p, np) {
+    for (int e = 0; e < E; e++) {
+      const int q = src[(size_t)e * np + p];
+      coef[(size_t)e * np + p] = q >= 0 ? lu[q] : 0.0;
+    }
+    dg[p] = rowid[p] >= 0 ? lu[diag[rowid[p]]] : 1.0;
+  }
+}
+
 // y = y - sigma x, skipped like the products
 __global__ __launch_bounds__(KS_BLOCK) void k_shift_gated(int n, const double *__restrict__ x, double *__restrict__ y,
                                                          double sigma, const ksp_state *S, int skip_sconv) {
@@ -530,14 +635,50 @@ struct ks_ilu_s {
   unsigned long long *d_slot = nullptr;   // [n][2] published values of the triangular solves
   unsigned epoch = 0;
   const int32_t *d_rowptr = nullptr, *d_colidx = nullptr;   // the operator's pattern (borrowed)
+  // one factor in level order for k_ilu0_levels (nsteps 0: k_ilu0_sf takes it)
+  struct lvl {
+    int nsteps = 0, nt = 0, E = 0, ring = 0;
+    int32_t *d_idx = nullptr;      // rowid[np], dep[E][np], src[E][np]
+    double *d_val = nullptr;       // dg[np], then coef[E][np]
+  } lo, up;
+  int32_t *d_lvl = nullptr;        // both layouts' d_idx
 };
 
 namespace {
 
+#define KS_ILU_EMAX 4          // entries a row in the level-ordered layout
+#define KS_ILU_RING 16384      // solved values held in LDS (128 KB), at most
+
+template <bool LOWER, int E, int NT>
+void launch_levels(ks_ctx ctx, const ks_ilu_s::lvl &L, double *y, const ksp_state *S, int skip_sconv) {
+  const int np = L.nsteps * NT;
+  hipLaunchKernelGGL((k_ilu0_levels<LOWER, E, NT>), dim3(1), dim3(NT), sizeof(double) * (L.ring + 1), ctx->stream,
+                     L.nsteps, L.ring, (const int32_t *)L.d_idx, (const int32_t *)L.d_idx + np,
+                     (const double *)L.d_val + np, (const double *)L.d_val, y, S, skip_sconv);
+}
+template <bool LOWER>
+void apply_levels(ks_ctx ctx, const ks_ilu_s::lvl &L, double *y, const ksp_state *S, int skip_sconv) {
+  if (L.nt == 256) {
+    if (L.E == 2) launch_levels<LOWER, 2, 256>(ctx, L, y, S, skip_sconv);
+    else launch_levels<LOWER, 4, 256>(ctx, L, y, S, skip_sconv);
+  } else if (L.nt == 512) {
+    if (L.E == 2) launch_levels<LOWER, 2, 512>(ctx, L, y, S, skip_sconv);
+    else launch_levels<LOWER, 4, 512>(ctx, L, y, S, skip_sconv);
+  } else {   // 1024 threads leave 128 VGPRs, enough for two entries a row
+    launch_levels<LOWER, 2, 1024>(ctx, L, y, S, skip_sconv);
+  }
+}
+
 // y = (L U)^-1 y on the context stream: two launches, the forward and the
-// backward solve, each a new epoch of the published values
+// backward solve, by levels where the factors have that layout, else each a
+// new epoch of the published values
 void ilu0_apply(ks_ctx ctx, ks_ilu M, double *y, const ksp_state *S, int skip_sconv) {
   const int blocks = (M->n + KS_WAVES - 1) / KS_WAVES;
+  if (M->lo.nsteps && M->up.nsteps) {
+    apply_levels<true>(ctx, M->lo, y, S, skip_sconv);
+    apply_levels<false>(ctx, M->up, y, S, skip_sconv);
+    return;
+  }
   M->epoch += 1;
   hipLaunchKernelGGL(k_ilu0_sf<true>, dim3(blocks), dim3(KS_BLOCK), 0, ctx->stream, M->n, M->d_rowptr,
                      M->d_colidx, (const int32_t *)M->d_diag, (const double *)M->d_lu, y, M->d_slot, M->epoch,
@@ -558,6 +699,79 @@ void group_levels(const std::vector<int> &lev, std::vector<int32_t> &rows, std::
   std::vector<int> fill(ptr.begin(), ptr.end() - 1);
   rows.resize(lev.size());
   for (size_t i = 0; i < lev.size(); i++) rows[fill[lev[i]]++] = (int32_t)i;
+}
+
+// The level-ordered layout of one factor (entries q0(i) .. q1(i)-1 of row i),
+// appended to idx: which row, which ring slots and which factor entries stand in
+// every slot.  Returns false, and the factors keep k_ilu0_sf, where a row has
+// more than KS_ILU_EMAX entries, a dependency lies further back than the ring,
+// or the levels are so wide that the steps outnumber them KS_ILU_STEPS times
+// (k_ilu0_sf has the whole chip for them).  A BiCGStab iteration (four
+// triangular solves), k_ilu0_sf / by levels: five-point grids 64 x 63 592 / 160
+// us, 128 x 127 1449 / 331, 256 x 255 7.1 / 0.84 ms, 512 x 511 48.9 / 3.0 ms;
+// seven-point grids 16^3 283 / 114 us, 64^3 (levels 1380 rows wide on average)
+// 10.7 / 2.9 ms; a tridiagonal matrix of 20,000 rows 84.8 / 20.2 ms.
+#define KS_ILU_STEPS 4
+template <typename Q0, typename Q1>
+bool level_layout(int n, const std::vector<int32_t> &rows, const std::vector<int> &ptr, const std::vector<int32_t> &ci,
+                  Q0 q0, Q1 q1, ks_ilu_s::lvl &L, std::vector<int32_t> &idx) {
+  const int nl = (int)ptr.size() - 1;
+  int emax = 0, wmax = 0;
+  for (int i = 0; i < n; i++) emax = std::max(emax, (int)(q1(i) - q0(i)));
+  for (int l = 0; l < nl; l++) wmax = std::max(wmax, ptr[l + 1] - ptr[l]);
+  if (emax > KS_ILU_EMAX) return false;
+  const int E = emax <= 2 ? 2 : KS_ILU_EMAX, nt = wmax <= 256 ? 256 : (wmax <= 512 || E > 2 ? 512 : 1024);
+  int64_t steps = 0;
+  for (int l = 0; l < nl; l++) steps += (ptr[l + 1] - ptr[l] + nt - 1) / nt;
+  if (steps > (int64_t)KS_ILU_STEPS * nl || steps * nt * E >= (1 << 29)) return false;
+  const int np = (int)steps * nt;
+  std::vector<int> pos(n);
+  const size_t at = idx.size();
+  idx.resize(at + (size_t)np * (2 * E + 1), -1);
+  int32_t *id = idx.data() + at, *dep = id + np, *src = dep + (size_t)np * E;
+  int s = 0, ring = nt;
+  for (int l = 0; l < nl; l++) {
+    for (int k = ptr[l]; k < ptr[l + 1]; k++) {
+      const int i = rows[k], p = s * nt + (k - ptr[l]), end = (p / nt + 1) * nt;
+      pos[i] = p;
+      id[p] = i;
+      size_t e = p;
+      for (int32_t q = q0(i); q < q1(i); q++, e += np) {
+        const int back = end - pos[ci[q]];   // slots written from the entry's value to the end of this step
+        while (ring < back && ring <= KS_ILU_RING) ring *= 2;
+        if (ring > KS_ILU_RING) return false;
+        dep[e] = pos[ci[q]];
+        src[e] = q;
+      }
+    }
+    s += (ptr[l + 1] - ptr[l] + nt - 1) / nt;
+  }
+  for (size_t k = 0; k < (size_t)np * E; k++) dep[k] = dep[k] < 0 ? ring : (dep[k] & (ring - 1));
+  L.nsteps = (int)steps;
+  L.nt = nt;
+  L.E = E;
+  L.ring = ring;
+  return true;
+}
+
+// uploads both layouts and packs the factors' values
+int levels_pack(ks_ctx ctx, ks_ilu M, const std::vector<int32_t> &idx) {
+  size_t off = 0, val = 0;
+  KS_TRY(ks_malloc((void **)&M->d_lvl, sizeof(int32_t) * idx.size()));
+  KS_HIP(hipMemcpyAsync(M->d_lvl, idx.data(), sizeof(int32_t) * idx.size(), hipMemcpyHostToDevice, ctx->stream));
+  for (ks_ilu_s::lvl *L : {&M->lo, &M->up}) val += (size_t)L->nsteps * L->nt * (L->E + 1);
+  KS_TRY(ks_malloc((void **)&M->lo.d_val, sizeof(double) * val));
+  M->up.d_val = M->lo.d_val + (size_t)M->lo.nsteps * M->lo.nt * (M->lo.E + 1);
+  for (ks_ilu_s::lvl *L : {&M->lo, &M->up}) {
+    const int np = L->nsteps * L->nt;
+    L->d_idx = M->d_lvl + off;
+    off += (size_t)np * (2 * L->E + 1);
+    hipLaunchKernelGGL(k_ilu0_pack, dim3(ksp_blocks(np)), dim3(KS_BLOCK), 0, ctx->stream, np, L->E,
+                       (const int32_t *)L->d_idx + (size_t)np * (L->E + 1), (const int32_t *)L->d_idx,
+                       (const int32_t *)M->d_diag, (const double *)M->d_lu, L->d_val + np, L->d_val);
+  }
+  KS_HIP(hipGetLastError());
+  return KS_OK;
 }
 
 }  // namespace
@@ -595,7 +809,9 @@ int ks_ilu0_create(ks_ctx ctx, ks_csr A, double sigma, ks_ilu *out) {
     for (int32_t q = diag[i] + 1; q < rp[i + 1]; q++) lev[i] = lev[ci[q]] + 1 > lev[i] ? lev[ci[q]] + 1 : lev[i];
   group_levels(lev, urows, M->uptr);
   int e = KS_OK;
-  if (!e) e = ks_malloc((void **)&M->d_lrows, sizeof(int32_t) * n);
+  // the rows by level and the level starts
+  lrows.insert(lrows.end(), M->lptr.begin(), M->lptr.end());
+  if (!e) e = ks_malloc((void **)&M->d_lrows, sizeof(int32_t) * lrows.size());
   if (!e) e = ks_malloc((void **)&M->d_diag, sizeof(int32_t) * n);
   if (!e) e = ks_malloc((void **)&M->d_lu, sizeof(double) * (nnz > 0 ? nnz : 1));
   if (!e) e = ks_malloc((void **)&M->d_flag, sizeof(int));
@@ -606,18 +822,39 @@ int ks_ilu0_create(ks_ctx ctx, ks_csr A, double sigma, ks_ilu *out) {
     return e;
   }
   hipStream_t st = ctx->stream;
-  KS_HIP(hipMemcpyAsync(M->d_lrows, lrows.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice, st));
+  KS_HIP(hipMemcpyAsync(M->d_lrows, lrows.data(), sizeof(int32_t) * lrows.size(), hipMemcpyHostToDevice, st));
   KS_HIP(hipMemcpyAsync(M->d_diag, diag.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice, st));
   KS_TRY(ks_memset_zero(ctx, M->d_flag, sizeof(int)));
   hipLaunchKernelGGL(k_ilu0_init, dim3(ksp_blocks(n)), dim3(KS_BLOCK), 0, st, A->d_rowptr, A->d_colidx,
                      (const double *)A->d_val, n, sigma, M->d_lu);
-  for (size_t l = 0; l + 1 < M->lptr.size(); l++) {
-    const int cnt = M->lptr[l + 1] - M->lptr[l];
-    hipLaunchKernelGGL(k_ilu0_factor_level, dim3((cnt + 63) / 64), dim3(64), 0, st,
-                       (const int32_t *)M->d_lrows + M->lptr[l], cnt, A->d_rowptr, A->d_colidx,
-                       (const int32_t *)M->d_diag, M->d_lu, M->d_flag);
+  const int nlev = (int)M->lptr.size() - 1;
+  int wmax = 0;
+  for (int l = 0; l < nlev; l++) wmax = std::max(wmax, M->lptr[l + 1] - M->lptr[l]);
+  if (wmax <= KS_ILU_WG) {
+    hipLaunchKernelGGL(k_ilu0_factor, dim3(1), dim3(KS_ILU_WG), 0, st, (const int32_t *)M->d_lrows,
+                       (const int32_t *)M->d_lrows + n, nlev, A->d_rowptr, A->d_colidx, (const int32_t *)M->d_diag,
+                       M->d_lu, M->d_flag);
+  } else {
+    for (int l = 0; l < nlev; l++) {
+      const int cnt = M->lptr[l + 1] - M->lptr[l];
+      hipLaunchKernelGGL(k_ilu0_factor_level, dim3((cnt + 63) / 64), dim3(64), 0, st,
+                         (const int32_t *)M->d_lrows + M->lptr[l], cnt, A->d_rowptr, A->d_colidx,
+                         (const int32_t *)M->d_diag, M->d_lu, M->d_flag);
+    }
   }
   KS_HIP(hipGetLastError());
+  // the level-ordered layouts, made while the device factors
+  std::vector<int32_t> idx;
+  const bool by_levels =
+      level_layout(n, lrows, M->lptr, ci, [&](int i) { return rp[i]; }, [&](int i) { return diag[i]; }, M->lo, idx) &&
+      level_layout(n, urows, M->uptr, ci, [&](int i) { return diag[i] + 1; }, [&](int i) { return rp[i + 1]; }, M->up,
+                   idx);
+  if (!by_levels) M->lo.nsteps = M->up.nsteps = 0;
+  else if ((e = levels_pack(ctx, M, idx))) {
+    (void)hipStreamSynchronize(st);
+    ks_ilu0_destroy(M);
+    return e;
+  }
   // the last pivot, and a zero pivot met on the way
   int flag = 0;
   double ulast = 0.0;
@@ -640,6 +877,8 @@ int ks_ilu0_destroy(ks_ilu M) {
   if (M->d_diag) (void)ks_free(M->d_diag);
   if (M->d_lu) (void)ks_free(M->d_lu);
   if (M->d_flag) (void)ks_free(M->d_flag);
+  if (M->d_lvl) (void)ks_free(M->d_lvl);
+  if (M->lo.d_val) (void)ks_free(M->lo.d_val);
   delete M;
   return KS_OK;
 }
