@@ -220,6 +220,20 @@ extern "C" int *ks_prof_begin(ks_ctx ctx, int cls, double bytes, double flops, b
 extern "C" void ks_prof_end(ks_ctx ctx);
 
 // ---------------------------------------------------------------- device helpers
+// Workgroups go to the 8 XCDs round-robin (workgroup i to XCD i mod 8), each
+// XCD with its own L2.  Row block ks_xcd_block(i) gives XCD x a contiguous eighth
+// of the row blocks, so the x entries a block gathers from neighbouring rows
+// (a stencil's +-1, +-nx, +-nx*ny) are mostly in the L2 its XCD already filled.
+// A bijection on [0, nb) for any nb.
+#ifndef KS_SPMV_XCD
+#define KS_SPMV_XCD 1
+#endif
+__device__ __forceinline__ int ks_xcd_block(int i, int nb) {
+  if (!KS_SPMV_XCD) return i;
+  const int q = nb >> 3, r = nb & 7, x = i & 7, j = i >> 3;
+  return x < r ? x * (q + 1) + j : r * (q + 1) + (x - r) * q + j;
+}
+
 // lane k's value of v, to every lane (k wave-uniform), as two 32-bit readlanes
 __device__ __forceinline__ double ks_readlane_f64(double v, int k) {
   const long long bits = __double_as_longlong(v);
