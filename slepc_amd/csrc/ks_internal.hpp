@@ -260,15 +260,67 @@ __device__ __forceinline__ double ks_pub_f64(unsigned long long lo, unsigned lon
   return __longlong_as_double((long long)(((hi & 0xffffffffull) << 32) | (lo & 0xffffffffull)));
 }
 
+// Exchanges between lanes l and l ^ OFF without the LDS pipe (a __shfl_xor is a
+// ds_bpermute, about 100 cycles; these are a few).  32 and 16 use gfx950's lane
+// swaps: ks_lane_swap leaves {a of the lower half, b of the lower half} in a and
+// {a of the upper half, b of the upper half} in b, so a + b holds, in the lower
+// lanes, a's sum over the pair and, in the upper lanes, b's.
+template <int OFF>
+__device__ __forceinline__ void ks_lane_swap(double &a, double &b) {
+  static_assert(OFF == 32 || OFF == 16, "lane swaps exist for 32 and 16");
+  const long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+  typedef unsigned u2 __attribute__((ext_vector_type(2)));
+  u2 lo, hi;
+  if constexpr (OFF == 32) {
+    lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+    hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+  } else {
+    lo = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+    hi = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+  }
+  a = __longlong_as_double(((long long)hi.x << 32) | lo.x);
+  b = __longlong_as_double(((long long)hi.y << 32) | lo.y);
+}
+template <int OFF>
+__device__ __forceinline__ int ks_lane_xor32(int v) {
+  static_assert(OFF == 8 || OFF == 4 || OFF == 2 || OFF == 1, "within a row of 16 lanes");
+  if constexpr (OFF == 8) return __builtin_amdgcn_update_dpp(0, v, 0x128, 0xf, 0xf, false);         // row_ror:8
+  else if constexpr (OFF == 4) {
+    const int t = __builtin_amdgcn_update_dpp(0, v, 0x104, 0xf, 0x5, false);                        // row_shl:4
+    return __builtin_amdgcn_update_dpp(t, v, 0x114, 0xf, 0xa, false);                               // row_shr:4
+  } else if constexpr (OFF == 2) return __builtin_amdgcn_update_dpp(0, v, 0x4e, 0xf, 0xf, false);   // quad_perm 2301
+  else return __builtin_amdgcn_update_dpp(0, v, 0xb1, 0xf, 0xf, false);                             // quad_perm 1032
+}
+// lane l ^ OFF's value
+template <int OFF>
+__device__ __forceinline__ double ks_lane_xor(double v) {
+  const long long x = __double_as_longlong(v);
+  const int lo = ks_lane_xor32<OFF>((int)x), hi = ks_lane_xor32<OFF>((int)(x >> 32));
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// v plus lane l ^ OFF's value
+template <int OFF>
+__device__ __forceinline__ double ks_lane_xor_add(double v) {
+  if constexpr (OFF >= 16) {
+    double a = v, b = v;
+    ks_lane_swap<OFF>(a, b);
+    return a + b;
+  } else return v + ks_lane_xor<OFF>(v);
+}
+
+// the sum over the wave's 64 lanes, in every lane
 __device__ __forceinline__ double ks_wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
+  v = ks_lane_xor_add<32>(v);
+  v = ks_lane_xor_add<16>(v);
+  v = ks_lane_xor_add<8>(v);
+  v = ks_lane_xor_add<4>(v);
+  v = ks_lane_xor_add<2>(v);
+  return ks_lane_xor_add<1>(v);
 }
 
 // Wave sums of M values per lane by recursive halving: at each step the lanes
 // of an xor pair keep opposite halves of their values and add the partner's
-// copy of the half they keep, so M values cost about M + 3 log2(64) shuffles
+// copy of the half they keep, so M values cost about M + 3 log2(64) exchanges
 // instead of 6 M.  While M stays even the halving continues (offsets 32, 16,
 // ...); the values left are then summed over the remaining lane bits.  On
 // return v[i] of lane l holds the wave total of value ks_multi_sum<M>::index(l, i).
@@ -277,21 +329,27 @@ template <int M, int OFF>
 struct ks_multi_halve {
   // every index below is a compile-time constant, so v stays in registers
   __device__ static __forceinline__ void run(double *v, int lane) {
-    if constexpr (M % 2 == 0 && OFF >= 1) {
-      constexpr int half = M / 2;
-      const bool up = (lane & OFF) != 0;
+    if constexpr (OFF >= 1) {
+      if constexpr (M % 2 == 0) {
+        constexpr int half = M / 2;
 #pragma unroll
-      for (int i = 0; i < half; i++) {
-        const double keep = up ? v[half + i] : v[i];
-        const double give = up ? v[i] : v[half + i];
-        v[i] = keep + __shfl_xor(give, OFF, 64);
+        for (int i = 0; i < half; i++) {
+          if constexpr (OFF >= 16) {
+            ks_lane_swap<OFF>(v[i], v[half + i]);
+            v[i] += v[half + i];
+          } else {
+            const bool up = (lane & OFF) != 0;
+            const double keep = up ? v[half + i] : v[i];
+            const double give = up ? v[i] : v[half + i];
+            v[i] = keep + ks_lane_xor<OFF>(give);
+          }
+        }
+        ks_multi_halve<half, OFF / 2>::run(v, lane);
+      } else {
+#pragma unroll
+        for (int i = 0; i < M; i++) v[i] = ks_lane_xor_add<OFF>(v[i]);
+        ks_multi_halve<M, OFF / 2>::run(v, lane);   // M stays odd
       }
-      ks_multi_halve<half, OFF / 2>::run(v, lane);
-    } else {
-#pragma unroll
-      for (int off = OFF; off > 0; off >>= 1)
-#pragma unroll
-        for (int i = 0; i < M; i++) v[i] += __shfl_xor(v[i], off, 64);
     }
   }
 };
