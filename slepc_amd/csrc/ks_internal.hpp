@@ -98,6 +98,9 @@ struct ks_ctx_s {
   double *d_scalar = nullptr;      // small device scratch (norm results)
   double *h_scalar = nullptr;      // pinned host scratch
   ks_status *h_status = nullptr;   // pinned mirror of d_status, filled by ks_status_post
+  // a call's workspace, kept for the next call on the context (ks_ws_take)
+  void *d_ws = nullptr;
+  size_t ws_bytes = 0;
   // profiling
   bool prof = false;
   unsigned prof_mask = ~0u;   // classes that get events while prof is on
@@ -172,6 +175,15 @@ struct ks_csr_s {
   int32_t *d_rowptr = nullptr, *d_colidx = nullptr, *d_blk = nullptr;
   void *d_val = nullptr;
 };
+
+// A workspace for one call on ctx: while no pool is current, the context's own
+// (kept up to KS_WS_KEEP bytes: allocating and freeing 75 MB costs a call about
+// 0.5 ms), else a block of the pool.  A call takes at most one and has waited for
+// the stream, or enqueues nothing after its own work that uses it, when it gives
+// it back.
+#define KS_WS_KEEP ((size_t)256 << 20)
+int ks_ws_take(ks_ctx ctx, size_t bytes, void **p);
+void ks_ws_give(ks_ctx ctx, void *p);
 
 // ---------------------------------------------------------------- grouped launches (serving)
 #define KS_GROUP_MAX 16   // solves per grouped launch

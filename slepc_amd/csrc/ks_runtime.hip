@@ -133,6 +133,7 @@ int ks_ctx_destroy(ks_ctx c) {
   (void)hipFree(c->d_gpartial);
   if (c->d_finpub) (void)hipFree(c->d_finpub);
   if (c->d_coef1) (void)hipFree(c->d_coef1);
+  if (c->d_ws) (void)hipFree(c->d_ws);
   (void)hipFree(c->d_counters);
   (void)hipFree(c->d_scalar);
   if (c->d_ran) (void)hipFree(c->d_ran);
@@ -218,6 +219,37 @@ int ks_host_free(void *ptr) {
   KS_HIP(hipHostFree(ptr));
   return KS_OK;
 }
+
+}  // extern "C"
+
+int ks_ws_take(ks_ctx c, size_t bytes, void **p) {
+  *p = nullptr;
+  if (g_pool_current) return ks_malloc(p, bytes);
+  if (c->ws_bytes < bytes) {
+    KS_HIP(hipStreamSynchronize(c->stream));   // earlier work on the old block
+    if (c->d_ws) (void)hipFree(c->d_ws);
+    c->d_ws = nullptr;
+    c->ws_bytes = 0;
+    int e = ks_malloc(&c->d_ws, bytes);
+    if (e) return e;
+    c->ws_bytes = bytes;
+  }
+  *p = c->d_ws;
+  return KS_OK;
+}
+
+void ks_ws_give(ks_ctx c, void *p) {
+  if (!p) return;
+  if (p != c->d_ws) {
+    (void)ks_free(p);
+  } else if (c->ws_bytes > KS_WS_KEEP) {
+    (void)hipFree(c->d_ws);
+    c->d_ws = nullptr;
+    c->ws_bytes = 0;
+  }
+}
+
+extern "C" {
 
 /* ---------------------------------------------------------------- pools */
 int ks_pool_create(ks_pool *out, size_t dev_bytes, size_t host_bytes) {
