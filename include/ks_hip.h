@@ -261,7 +261,7 @@ int ks_bv_orthonormalize_column_noalloc(void *stream, ks_prec prec, int n, void 
    then runs ks_bv_orthonormalize_resume for that column and enqueues the rest
    of the expansion again; the result is bit for bit that of
    ks_bv_orthonormalize_column.  Other refinement types, safe mode, scale = 0
-   and the LDS sweeps (k > 128) fall back to the full sequence. */
+   and columns of 4 GiB and more fall back to the full sequence. */
 int ks_bv_orthonormalize_column_lean(ks_ctx ctx, ks_prec prec, int n, void *V, int ld, int k, double *d_buf,
                                      int ldbuf, int hcol, int col, ks_refine refine, double eta, int scale,
                                      int safe);

@@ -576,25 +576,25 @@ __global__ __launch_bounds__(KS_BLOCK) void k_gs_reg(const T *__restrict__ V, lo
 // pass used, then applies this pass's coefficients to it.
 // REFORM: the sweep can take defer == 2 (its extra sums cost registers, so only
 // the launches that may follow a deferred pass are built with it).
-template <typename T, int CW, bool FUSED, int RPL, bool PAIR, bool REFORM = false>
+template <typename T, int CW, bool FUSED, int RPL, bool PAIR, bool REFORM = false, int NWV = KS_WAVES,
+          typename AT = typename acc_t<T>::type>   // FP32 data: FP32 products and per-thread sums
 __device__ __forceinline__ void gs_split_block(int b, int nb, const T *__restrict__ V, long ld, int k,
                                                T *__restrict__ w, int n, int rpb, const double *__restrict__ cbuf,
                                                double *__restrict__ partial, double wscale, int defer = 0,
                                                const double *__restrict__ coef1 = nullptr) {
   static_assert(!PAIR || (sizeof(T) == 4 && RPL == 2), "row pairs are two adjacent FP32 rows");
-  using AT = typename acc_t<T>::type;   // FP32 data: FP32 products and per-thread sums
   constexpr int STEP = 64 * RPL;        // rows per step; each lane takes RPL of them
-  __shared__ AT coef[KS_WAVES * CW];
-  __shared__ AT red[2][KS_WAVES][STEP];
-  __shared__ AT coefp[REFORM ? KS_WAVES * CW : 1];          // coef1, when defer == 2
-  __shared__ AT redp[REFORM ? 2 : 1][KS_WAVES][REFORM ? STEP : 1];
+  __shared__ AT coef[NWV * CW];
+  __shared__ AT red[2][NWV][STEP];
+  __shared__ AT coefp[REFORM ? NWV * CW : 1];          // coef1, when defer == 2
+  __shared__ AT redp[REFORM ? 2 : 1][NWV][REFORM ? STEP : 1];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform: column guards are scalar branches
   const int c0 = wave * CW;
   // this lane's q-th row of a step: adjacent pairs (one 8-byte load) or 64 apart
   auto loff = [&](int q) { return PAIR ? RPL * lane + q : 64 * q + lane; };
   if (FUSED)
-    for (int c = tid; c < KS_WAVES * CW; c += KS_BLOCK) {
+    for (int c = tid; c < NWV * CW; c += 64 * NWV) {
       coef[c] = (AT)(c < k ? cbuf[c] : 0.0);
       if (REFORM && defer == 2) coefp[c] = (AT)(c < k ? coef1[c] : 0.0);
     }
@@ -664,15 +664,28 @@ __device__ __forceinline__ void gs_split_block(int b, int nb, const T *__restric
         const int r = loff(q);
         const unsigned i = i0 + r;
         AT base = wi[q];
-        if (REFORM && defer == 2)   // the previous pass's vector, as that pass formed it
-          base = (AT)(T)(base - (((redp[buf][0][r] + redp[buf][1][r]) + redp[buf][2][r]) + redp[buf][3][r]));
-        const AT tot = ((red[buf][0][r] + red[buf][1][r]) + red[buf][2][r]) + red[buf][3][r];
+        if (REFORM && defer == 2) {   // the previous pass's vector, as that pass formed it
+          AT prev = redp[buf][0][r];
+#pragma unroll
+          for (int x = 1; x < NWV; x++) prev += redp[buf][x][r];
+          base = (AT)(T)(base - prev);
+        }
+        AT tot = red[buf][0][r];
+#pragma unroll
+        for (int x = 1; x < NWV; x++) tot += red[buf][x][r];
         const T t = (T)(base - tot);
         wi[q] = i < r1 ? (AT)t : (AT)0;
         // the final pass of a column stores it normalized, rounded as k_scale_status would
         if (defer != 1 && wave == 0 && i < r1) w[i] = wscale == 1.0 ? t : (T)((AT)t * (AT)wscale);
       }
       buf ^= 1;
+      // FP32 values multiplied in FP64: converted again for the dots, not kept
+      // converted across the barrier (twice the registers, and scratch)
+      if constexpr (sizeof(T) < sizeof(AT))
+#pragma unroll
+        for (int q = 0; q < RPL; q++)
+#pragma unroll
+          for (int u = 0; u < CW; u++) asm volatile("" : "+v"(v[q][u]));
     }
 #pragma unroll
     for (int q = 0; q < RPL; q++) {
@@ -729,6 +742,25 @@ __global__ __launch_bounds__(KS_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) v
   gs_split_block<T, CW, FUSED, RPL, PAIR, REFORM>(blockIdx.x, gridDim.x, V, ld, k, w, n, rpb, cbuf, partial,
                                                   gs_prescale<FUSED>(st, col, pass), gs_defer<FUSED>(st, col, pass),
                                                   coef1);
+}
+
+// The same sweep for more than KS_GS_SPLITMAX columns: eight wavefronts split
+// them, so CW (and the registers of a thread) stays at most 40.  FP32 data is
+// multiplied and summed in FP64, as the LDS-staged kernel does.  No pass defers
+// its store: the vector is less than a hundredth of what a sweep reads here, and
+// the re-forming sums cost as much or more (a column of n = 405,224: k = 130 245 us
+// against 256 with deferral, k = 200 385 and 391, k = 310 580 and 643).
+#define KS_GS_WIDE_WAVES 8
+template <typename T, int CW, bool FUSED, bool PAIR>
+__global__ __launch_bounds__(64 * KS_GS_WIDE_WAVES) void k_gs_wide(const T *__restrict__ V, long ld, int k,
+                                                                  T *__restrict__ w, int n, int rpb,
+                                                                  const double *__restrict__ cbuf,
+                                                                  double *__restrict__ partial, const ks_status *st,
+                                                                  int col, int pass, int *ran) {
+  if (!gs_pass_gate<FUSED>(st, col, pass)) return;
+  if (ran && blockIdx.x == 0 && threadIdx.x == 0) *ran = 1;
+  gs_split_block<T, CW, FUSED, PAIR ? 2 : 1, PAIR, false, KS_GS_WIDE_WAVES, double>(
+      blockIdx.x, gridDim.x, V, ld, k, w, n, rpb, cbuf, partial, gs_prescale<FUSED>(st, col, pass));
 }
 
 // The finish of a Gram-Schmidt pass: a separate launch, ordered by the stream
@@ -1402,6 +1434,7 @@ struct gs_geom {
   size_t lds;
   int kc;   // > 0: register-resident kernel for up to kc columns
   int cw;   // > 0: column-split kernel, cw columns per wavefront
+  int wide; // column-split over eight wavefronts
   int pair; // column-split on FP32 data with two rows per lane (even ld, aligned)
   int rpl;  // column-split on FP64 data: rows per lane per step (2: two loads 64 rows apart)
 };
@@ -1409,6 +1442,7 @@ struct gs_geom {
 int gs_geometry(int n, int k, size_t esize, gs_geom *g) {
   g->kc = 0;
   g->cw = 0;
+  g->wide = 0;
   g->pair = 0;
   g->rpl = 1;
   if (k <= KS_GS_REGMAX && (uint64_t)n * esize < (1ull << 32)) {
@@ -1437,6 +1471,28 @@ int gs_geometry(int n, int k, size_t esize, gs_geom *g) {
     const long nb = tiles < cap ? tiles : cap;
     const long tpb = (tiles + nb - 1) / nb;
     g->cpb = (int)(tpb * step);                                         // rows per workgroup
+    g->nb = (int)((n + (long)g->cpb - 1) / g->cpb);
+    g->R = 0;
+    g->tsub = 0;
+    g->lds = 0;
+    return KS_OK;
+  }
+  // wider bases: the LDS-staged kernel only where a row's offset needs 64 bits.
+  // A column (three sweeps), LDS-staged / split: n = 405,224 FP64 k = 130 329 / 245
+  // us, k = 200 627 / 385 (5.2-5.9 TB/s), k = 310 807 / 580; FP32 k = 200 1222 / 227;
+  // n = 5,000 k = 200 44 / 42.  1024 workgroups instead of 512: k = 200 416 us.
+  if ((uint64_t)n * esize < (1ull << 32)) {
+    const int per = (k + KS_GS_WIDE_WAVES - 1) / KS_GS_WIDE_WAVES;
+    static const int cws[] = {20, 24, 28, 32, 40};
+    static_assert(40 * KS_GS_WIDE_WAVES >= KS_MAX_COLS, "every width has a sweep");
+    for (int c : cws)
+      if (per <= c) { g->cw = c; break; }
+    g->wide = 1;
+    const long step = esize == 4 ? 128 : 64;                            // rows per workgroup step, even
+    const long tiles = (n + step - 1) / step;
+    const long nb = tiles < KS_GS_WIDE_BLOCKS ? tiles : KS_GS_WIDE_BLOCKS;
+    const long tpb = (tiles + nb - 1) / nb;
+    g->cpb = (int)(tpb * step);
     g->nb = (int)((n + (long)g->cpb - 1) / g->cpb);
     g->R = 0;
     g->tsub = 0;
@@ -1489,9 +1545,30 @@ void launch_split(ks_ctx ctx, const gs_geom &g, const T *V, long ld, int k, T *w
 }
 
 template <typename T, bool FUSED>
+void launch_wide(ks_ctx ctx, const gs_geom &g, const T *V, long ld, int k, T *w, int n, const double *cbuf, int col,
+                 int pass, int *ran) {
+  dim3 grid(g.nb), block(64 * KS_GS_WIDE_WAVES);
+#define KS_GSW_CASE(CC)                                                                                          \
+  case CC:                                                                                                       \
+    if (g.pair)                                                                                                  \
+      hipLaunchKernelGGL((k_gs_wide<T, CC, FUSED, sizeof(T) == 4>), grid, block, 0, ctx->stream, V, ld, k, w, n, \
+                         g.cpb, cbuf, ctx->d_partial, ctx->d_status, col, pass, ran);                            \
+    else                                                                                                         \
+      hipLaunchKernelGGL((k_gs_wide<T, CC, FUSED, false>), grid, block, 0, ctx->stream, V, ld, k, w, n, g.cpb,   \
+                         cbuf, ctx->d_partial, ctx->d_status, col, pass, ran);                                   \
+    break;
+  switch (g.cw) { KS_GSW_CASE(20) KS_GSW_CASE(24) KS_GSW_CASE(28) KS_GSW_CASE(32) KS_GSW_CASE(40) }
+#undef KS_GSW_CASE
+}
+
+template <typename T, bool FUSED>
 void launch_gs(ks_ctx ctx, const gs_geom &g, const T *V, long ld, int k, T *w, int n, const double *cbuf, int col,
                int pass, int *ran) {
   dim3 grid(g.nb), block(KS_BLOCK);
+  if (g.wide) {
+    launch_wide<T, FUSED>(ctx, g, V, ld, k, w, n, cbuf, col, pass, ran);
+    return;
+  }
   if (g.cw) {
     if (FUSED && pass == 2)   // may follow a deferred first pass
       launch_split<T, FUSED, true>(ctx, g, V, ld, k, w, n, cbuf, col, pass, ran);
@@ -1523,7 +1600,7 @@ void launch_gs_fin(ks_ctx ctx, const gs_geom &g, int k, double *cbuf, double *hc
                    double eta, int do_scale, int safe, int halt_pass) {
   const double deftol = 10.0 * 2.220446049250313e-16;
   ks_prof_begin(ctx, KS_PROF_GS_FIN, (double)g.nb * (k + 1) * 8.0, (double)g.nb * (k + 1), false);
-  double *coef1 = g.cw ? ctx->d_coef1 : nullptr;   // deferred first-pass store: split sweeps only
+  double *coef1 = g.cw && !g.wide ? ctx->d_coef1 : nullptr;   // deferred first-pass store: split sweeps only
   if (ctx->d_finpub)
     hipLaunchKernelGGL((k_gs_fin_pub<FUSED>), dim3(k + 2), dim3(KS_FIN_BLOCK), 0, ctx->stream, ctx->d_partial, g.nb,
                        k, ctx->d_finpub, cbuf, hcol, ctx->d_status, col, pass, refine, eta, do_scale, safe, deftol,
@@ -1572,7 +1649,7 @@ int orthonormalize_t(ks_ctx ctx, int n, T *V, long ld, int k, double *buf, int l
   // follows) that pass is counted without its write -- it stores only in the
   // rare column it is also the last pass of -- and the next one with the
   // re-formed product's flops
-  const bool deferrable = g.cw && ctx->d_coef1 && !safe && refine != KS_REFINE_NEVER;
+  const bool deferrable = g.cw && !g.wide && ctx->d_coef1 && !safe && refine != KS_REFINE_NEVER;
   for (int p = p_first; p <= p_last; p++) {
     const double bytes = (p == 1 && deferrable ? k + 1.0 : k + 2.0) * n * s;
     const double flops = 2.0 * k * n + 2.0 * (k + 1.0) * n + (p == 2 && deferrable ? 2.0 * k * n : 0.0);
@@ -1675,8 +1752,8 @@ int ks_gs_split_geometry(int n, int k, int *cw, int *rpb, int *nb) {
   gs_geom g;
   int e = gs_geometry(n, k, sizeof(double), &g);
   if (e) return e;
-  if (!g.cw) {
-    // the grouped launches run the column-split sweep only; its geometry for this k
+  if (!g.cw || g.wide) {
+    // the grouped launches run the column-split sweep of four wavefronts only; its geometry for this k
     KS_CHECK(k <= KS_GS_SPLITMAX && (uint64_t)n * sizeof(double) < (1ull << 32), KS_ERR_RANGE,
              "grouped Gram-Schmidt supports up to %d columns (asked %d)", KS_GS_SPLITMAX, k);
     const int per = (k + KS_WAVES - 1) / KS_WAVES;
