@@ -270,6 +270,20 @@ int ks_bv_orthonormalize_column_lean(ks_ctx ctx, ks_prec prec, int n, void *V, i
    scaling, each gated on the device as in ks_bv_orthonormalize_column. */
 int ks_bv_orthonormalize_resume(ks_ctx ctx, ks_prec prec, int n, void *V, int ld, int k, double *d_buf, int ldbuf,
                                 int hcol, int col, ks_refine refine, double eta);
+/* Steps k..m-1 of an Arnoldi/Lanczos expansion (BVMatArnoldi / BVMatLanczos,
+   src/sys/classes/bv/interface/bvkrylov.c:88-97) in one launch, for small
+   problems: columns k+1..m after the nc constraint columns of V become A times
+   the column before them, orthonormalized against all columns before them
+   (as ks_bv_orthonormalize_column with scale = 1, safe = 0); column j's
+   coefficients and norm go to column j of d_buf.  The status must have been
+   reset; it reports breakdown and the last norm as after the launches.  *taken = 0
+   (and nothing enqueued) where the launches are the way: more than 192 row
+   blocks, a row longer than a row block, more than 128 columns, m >= n, events
+   or a capture on the context.  A status error of KS_ERR_TIMEOUT (its
+   workgroups could not run at the same time): expand again by the launches,
+   column k and those before it are as they were. */
+int ks_arnoldi_expand(ks_ctx ctx, ks_csr A, ks_prec prec, int n, void *V, int ld, int nc, int k, int m,
+                      double *d_buf, int ldbuf, ks_refine refine, double eta, int *taken);
 /* Reset the status for a new expansion (active=1, breakdown_col=-1). */
 int ks_status_reset(ks_ctx ctx);
 /* Copy the status to the host (synchronizes the stream). */

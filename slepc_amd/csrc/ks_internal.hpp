@@ -101,6 +101,8 @@ struct ks_ctx_s {
   double *d_scalar = nullptr;      // small device scratch (norm results)
   double *h_scalar = nullptr;      // pinned host scratch
   ks_status *h_status = nullptr;   // pinned mirror of d_status, filled by ks_status_post
+  unsigned long long *d_exp = nullptr;      // the exchange areas of ks_arnoldi_expand, and ...
+  unsigned exp_epoch = 0;                   // ... the next launch's first epoch
   // a call's workspace, kept for the next call on the context (ks_ws_take)
   void *d_ws = nullptr;
   size_t ws_bytes = 0;

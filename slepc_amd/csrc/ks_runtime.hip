@@ -134,6 +134,7 @@ int ks_ctx_destroy(ks_ctx c) {
   if (c->d_finpub) (void)hipFree(c->d_finpub);
   if (c->d_coef1) (void)hipFree(c->d_coef1);
   if (c->d_ws) (void)hipFree(c->d_ws);
+  if (c->d_exp) (void)hipFree(c->d_exp);
   (void)hipFree(c->d_counters);
   (void)hipFree(c->d_scalar);
   if (c->d_ran) (void)hipFree(c->d_ran);

@@ -43,6 +43,9 @@ typedef struct {
   PetscInt kry_k, kry_m;
   Mat kry_A;             /* the operator of the expansion in flight */
   PetscBool kry_posted;  /* status and buffer copied to pinned host memory in stream order */
+  PetscBool kry_fused;   /* the whole expansion went out as one launch (ks_arnoldi_expand) */
+  PetscBool fuse_not;    /* BVHIPKSSetOneLaunch */
+  PetscBool fuse_off;    /* such a launch's workgroups could not all run once: no more of them */
   int64_t resumes;       /* expansions a lean step stopped and the host resumed */
   /* grouped expansions (serving): the steps k..m-1 are enqueued by the server,
      step kry_j next, while kry_pending */
@@ -423,19 +426,46 @@ static PetscErrorCode KrylovSteps(BV V, Mat A, PetscInt j0, PetscInt m)
   return e;
 }
 
+/* the whole expansion as one launch where the kernel library takes it (small problems) */
+static PetscErrorCode KrylovFused(BV V, Mat A, PetscInt k, PetscInt m, PetscBool *done)
+{
+  BV_HIPKS *h = (BV_HIPKS *)V->data;
+  ks_csr csr;
+  double *dbuf;
+  int taken = 0;
+  *done = PETSC_FALSE;
+  if (h->fuse_off || h->fuse_not || !MatTypeIs(A, MATHIPCSR) || !A->data || SlepcAMDContext() != h->ctx || m > V->N - 1)
+    return PETSC_SUCCESS;
+  if (h->prec == SLEPC_AMD_F32) PetscCall(MatHIPCSRGetF32(A, &csr));
+  else csr = ((Mat_HIPCSR *)A->data)->csr;
+  if (!csr || ((Mat_HIPCSR *)A->data)->gate) return PETSC_SUCCESS;
+  PetscCall(BufferDevice(V, &dbuf));
+  KSCall(ks_arnoldi_expand(h->ctx, csr, kp(V), V->n, h->dV, V->ld, V->nc, k, m, dbuf, h->ncols,
+                           (ks_refine)V->orthog_ref, V->orthog_eta, &taken));
+  if (!taken) return PETSC_SUCCESS;
+  h->kry_fused = *done = PETSC_TRUE;
+  return BVHIPKSPostExpansion(V);
+}
+
 static PetscErrorCode BVMatKrylovBegin_HIPKS(BV V, Mat A, PetscInt k, PetscInt m)
 {
   BV_HIPKS *h = (BV_HIPKS *)V->data;
+  PetscBool done;
   KSCall(ks_status_reset(h->ctx));
   h->kry_posted = PETSC_FALSE;
   h->kry_k = k;
   h->kry_m = m;
   h->kry_A = A;
+  h->kry_fused = PETSC_FALSE;
   if (k < m && GroupEligible(V, A, m)) {
     h->kry_csr = ((Mat_HIPCSR *)A->data)->csr;
     h->kry_j = k;
     h->kry_pending = PETSC_TRUE;
     return PETSC_SUCCESS;
+  }
+  if (k < m) {
+    PetscCall(KrylovFused(V, A, k, m, &done));
+    if (done) return PETSC_SUCCESS;
   }
   return KrylovSteps(V, A, k, m);
 }
@@ -480,6 +510,13 @@ static PetscErrorCode BVMatKrylovEnd_HIPKS(BV V, PetscInt k, PetscInt *m, PetscR
   for (;;) {
     if (h->kry_posted) KSCall(ks_status_read(h->ctx, &st));
     else KSCall(ks_status_get(h->ctx, &st));
+    if (h->kry_fused && st.error == KS_ERR_TIMEOUT) {   /* its workgroups could not all run: the launches */
+      h->kry_fused = h->kry_posted = PETSC_FALSE;
+      h->fuse_off = PETSC_TRUE;
+      KSCall(ks_status_reset(h->ctx));
+      PetscCall(KrylovSteps(V, h->kry_A, h->kry_k, h->kry_m));
+      continue;
+    }
     PetscCall(StatusCheck(&st));
     if (st.halt_col < 0) break;
     /* a lean step stopped the expansion at column c: complete that column, then
@@ -673,6 +710,14 @@ PetscErrorCode BVHIPKSSetGrouped(BV bv, PetscBool grouped)
 {
   PetscCall(CheckHIPKS(bv));
   ((BV_HIPKS *)bv->data)->grouped = grouped;
+  return PETSC_SUCCESS;
+}
+
+/* whether expansions may go out as one launch (ks_arnoldi_expand); they do unless told otherwise */
+PetscErrorCode BVHIPKSSetOneLaunch(BV bv, PetscBool flg)
+{
+  PetscCall(CheckHIPKS(bv));
+  ((BV_HIPKS *)bv->data)->fuse_not = (PetscBool)!flg;
   return PETSC_SUCCESS;
 }
 

@@ -59,6 +59,11 @@ static PetscErrorCode EPSAllocateSolution(EPS eps, PetscInt extra)
   if (!strcmp(BVTypeName(V), BVHIPKS)) {
     PetscCall(BVHIPKSSetStepGraphs(V, ctx->step_graphs));
     PetscCall(BVHIPKSSetGrouped(V, ctx->grouped));
+    /* a harmonic restart's vector (u - V g) / gamma carries the expansion's rounding times
+       1 / gamma, some 1e6: results to a tolerance near that stay those of the launches' order
+       of sums (laplacian of 200 rows, target 1, tol 1e-10: eigenvalues good to 2e-11 in that
+       order, to 9e-11 in the one launch's, the other way round for other start vectors) */
+    PetscCall(BVHIPKSSetOneLaunch(V, (PetscBool)(eps->extraction != EPS_HARMONIC || eps->twosided)));
   }
   /* W: a basis like V for the two-sided variant (epssetup.c:726-731) */
   if (eps->W && (!eps->twosided || eps->W->m != requested || eps->W->n != eps->n || strcmp(eps->W->vtype, V->vtype)))

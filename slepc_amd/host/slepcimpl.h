@@ -317,6 +317,7 @@ PetscErrorCode BVHIPKSGetContext(BV bv, ks_ctx *ctx);
 PetscErrorCode BVHIPKSGetPasses(BV bv, int64_t *passes);
 PetscErrorCode BVHIPKSResetPasses(BV bv);
 PetscErrorCode BVHIPKSSetGrouped(BV bv, PetscBool grouped);
+PetscErrorCode BVHIPKSSetOneLaunch(BV bv, PetscBool flg);
 PetscErrorCode BVHIPKSGroupPending(BV bv, PetscBool *pending);
 PetscErrorCode BVHIPKSGroupMember(BV V, ks_group_member *mem);
 PetscErrorCode BVHIPKSGroupAdvance(BV V, PetscBool *finished);

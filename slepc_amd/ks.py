@@ -75,6 +75,7 @@ def lib():
             "ks_bv_orthonormalize_resume": [vp, i32, i32, vp, i32, i32, vp, i32, i32, i32, i32, dbl],
             "ks_bv_orthonormalize_column_noalloc": [vp, i32, i32, vp, i32, i32, vp, i32, i32, i32, i32, dbl,
                                                     i32, i32, vp],
+            "ks_arnoldi_expand": [vp, vp, i32, i32, vp, i32, i32, i32, i32, vp, i32, i32, dbl, C.POINTER(i32)],
             "ks_status_reset": [vp], "ks_status_get": [vp, C.POINTER(Status)],
             "ks_bv_scale": [vp, i32, i32, vp, dbl], "ks_bv_norm": [vp, i32, i32, vp, C.POINTER(dbl)],
             "ks_bv_axpy": [vp, i32, i32, dbl, vp, vp], "ks_bv_copy": [vp, i32, i32, vp, vp],
