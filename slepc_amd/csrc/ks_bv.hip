@@ -1284,101 +1284,193 @@ int dispatch_mip(ks_ctx ctx, T *V, long ld, int n, int K, const double *Q, int l
 }
 
 // ---------------------------------------------------------------- block dot (BVDot)
-// G = Y^T X for tall-skinny X (n x p) and Y (n x q), one 64 x 64 block of G
-// (rows i0.., columns j0..) per launch.  Workgroup b owns a contiguous range of
-// rows; per 32-row chunk it stages the 32 x 64 slices of X and Y in LDS with
-// coalesced column segments (rows past n and columns past p or q read a valid
-// element and are zeroed by a select, not a branch), and thread (ti, tj) of a
-// 16 x 16 grid accumulates the 4 x 4 entries G(i0+4ti.., j0+4tj..).  Partial
-// blocks go to partial[b][64*64]; k_gram_fin adds them in workgroup order.
-#define KS_GRAM_ROWS 32
+// G = Y^T X for tall-skinny X (n x p) and Y (n x q), one block of up to 64 x 64
+// entries of G (rows i0.., columns j0..) per launch, on v_mfma_f64_16x16x4f64
+// with the rows of X and Y as its k.  A wavefront owns rpw rows and all NY x NX
+// tiles of the block; lane l loads column l % 16 of a tile, rows l / 16 + 4 u,
+// straight into the operand registers (a load instruction covers 32 bytes of 16
+// columns), the next KS_GRAM_ROWS rows while the MFMAs of the current ones run.
+// Columns past p or q read the last one and land in entries that are not stored;
+// only a wavefront's last, incomplete rows are masked.  With SYM (Y is X, the
+// block on the diagonal) X is read once and the tiles above the diagonal, the
+// transposes of those below, are left out.  The workgroup's four blocks are added
+// in LDS ((0 + 2) + (1 + 3)) and go to partial[b], tile by tile in register
+// order; k_gram_fin adds the workgroups.
+// Bound by reading X and Y: 1,000,003 x 48 (X = Y) 449 -> 99 us (3.9 TB/s) against the
+// vector FP64 form over LDS that it took the place of, and the sum of 512 workgroups' blocks
+// 121 -> 6 us against a thread an entry; X, Y of 22,500 x 20: 21 + 85 -> 9 + 5 us.
+#define KS_GRAM_ROWS 16     // rows of a wavefront's step
 #define KS_GRAM_MAXB 512
-template <typename T>
-__global__ __launch_bounds__(KS_BLOCK) void k_gram(const T *__restrict__ X, long ldx, int p, const T *__restrict__ Y,
-                                                  long ldy, int q, int n, int rpb, int i0, int j0,
-                                                  double *__restrict__ partial) {
-  __shared__ double sX[KS_GRAM_ROWS][64];
-  __shared__ double sY[KS_GRAM_ROWS][64];
-  const int tid = threadIdx.x;
-  const int ti = tid >> 4, tj = tid & 15;
-  const int lr = tid & (KS_GRAM_ROWS - 1), lc = tid / KS_GRAM_ROWS;   // loader: row, first column
-  const long r0 = (long)blockIdx.x * rpb;
-  const long r1 = min((long)n, r0 + rpb);
-  double acc[4][4];
+template <typename T, int NY, int NX, bool SYM>
+__global__ __launch_bounds__(KS_BLOCK, 2) void k_gram(const T *__restrict__ X, long ldx, int p, const T *__restrict__ Y,
+                                                     long ldy, int q, int n, int rpw, int i0, int j0,
+                                                     double *__restrict__ partial) {
+  constexpr int NT = SYM ? NY * (NY + 1) / 2 : NY * NX, U = NT > 12 ? 2 : KS_GRAM_ROWS / 4, STEP = 4 * U;   // 4 x 4 tiles leave registers for 8 rows
+  __shared__ double sum[2][NT * 256];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lc = lane & 15, lk = lane >> 4;
+  const long r0 = min((long)n, (long)(blockIdx.x * KS_WAVES + wave) * rpw), r1 = min((long)n, r0 + rpw);
+  const T *xp[NX], *yp[NY];
 #pragma unroll
-  for (int a = 0; a < 4; a++)
+  for (int t = 0; t < NX; t++) xp[t] = X + (size_t)min(j0 + 16 * t + lc, p - 1) * ldx;
+  if (!SYM)
 #pragma unroll
-    for (int c = 0; c < 4; c++) acc[a][c] = 0.0;
-  for (long rb = r0; rb < r1; rb += KS_GRAM_ROWS) {
-    const long row = rb + lr;
-    const bool rok = row < r1;
-    const long rowc = rok ? row : r1 - 1;
-    double vx[8], vy[8];
+    for (int t = 0; t < NY; t++) yp[t] = Y + (size_t)min(i0 + 16 * t + lc, q - 1) * ldy;
+  v4d acc[NT];
 #pragma unroll
-    for (int u = 0; u < 8; u++) {
-      const int c = lc + 8 * u;
-      const int cx = min(j0 + c, p - 1), cy = min(i0 + c, q - 1);
-      vx[u] = (double)X[(size_t)cx * ldx + rowc];
-      vy[u] = (double)Y[(size_t)cy * ldy + rowc];
+  for (int t = 0; t < NT; t++) acc[t] = v4d{0.0, 0.0, 0.0, 0.0};
+  auto load = [&](long rb, T (&vx)[U][NX], T (&vy)[U][NY]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const long row = rb + 4 * u + lk;
+#pragma unroll
+      for (int t = 0; t < NX; t++) vx[u][t] = xp[t][row];
+      if (!SYM)
+#pragma unroll
+        for (int t = 0; t < NY; t++) vy[u][t] = yp[t][row];
     }
+  };
+  auto mac = [&](const T (&vx)[U][NX], const T (&vy)[U][NY]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      int t = 0;
+#pragma unroll
+      for (int a = 0; a < NY; a++)
+#pragma unroll
+        for (int c = 0; c < (SYM ? a + 1 : NX); c++, t++)
+          acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)(SYM ? vx[u][a % NX] : vy[u][a]), (double)vx[u][c], acc[t], 0, 0, 0);
+    }
+  };
+  const long rfull = r0 + (r1 - r0) / STEP * STEP;
+  T vx[U][NX], vy[U][NY];
+  if (r0 < rfull) load(r0, vx, vy);
+  for (long rb = r0; rb < rfull; rb += STEP) {
+    T nx[U][NX], ny[U][NY];
+    load(min(rb + STEP, rfull - STEP), nx, ny);   // the last step's again: not used
     __builtin_amdgcn_sched_barrier(0);
-    __syncthreads();   // the previous chunk's reads are done
+    mac(vx, vy);
 #pragma unroll
-    for (int u = 0; u < 8; u++) {
-      const int c = lc + 8 * u;
-      sX[lr][c] = (rok && j0 + c < p) ? vx[u] : 0.0;
-      sY[lr][c] = (rok && i0 + c < q) ? vy[u] : 0.0;
-    }
-    __syncthreads();
-#pragma unroll 4
-    for (int r = 0; r < KS_GRAM_ROWS; r++) {
-      double a[4], bb[4];
+    for (int u = 0; u < U; u++) {
 #pragma unroll
-      for (int u = 0; u < 4; u++) {
-        a[u] = sY[r][4 * ti + u];
-        bb[u] = sX[r][4 * tj + u];
-      }
+      for (int t = 0; t < NX; t++) vx[u][t] = nx[u][t];
+      if (!SYM)
 #pragma unroll
-      for (int u = 0; u < 4; u++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) acc[u][v] += a[u] * bb[v];
+        for (int t = 0; t < NY; t++) vy[u][t] = ny[u][t];
     }
   }
-  double *out = partial + (size_t)blockIdx.x * 4096;
+  if (rfull < r1) {
 #pragma unroll
-  for (int u = 0; u < 4; u++)
+    for (int u = 0; u < U; u++) {
+      const long row = rfull + 4 * u + lk, rowc = min(row, r1 - 1);
 #pragma unroll
-    for (int v = 0; v < 4; v++) out[(4 * ti + u) * 64 + 4 * tj + v] = acc[u][v];
+      for (int t = 0; t < NX; t++) {
+        const T v = xp[t][rowc];
+        vx[u][t] = row < r1 ? v : (T)0;
+      }
+      if (!SYM)
+#pragma unroll
+        for (int t = 0; t < NY; t++) {
+          const T v = yp[t][rowc];
+          vy[u][t] = row < r1 ? v : (T)0;
+        }
+    }
+    mac(vx, vy);
+  }
+  auto put = [&](double *o) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) o[(4 * t + e) * 64 + lane] = acc[t][e];
+  };
+  auto add = [&](const double *o) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) acc[t][e] += o[(4 * t + e) * 64 + lane];
+  };
+  if (wave >= 2) put(sum[wave - 2]);
+  __syncthreads();
+  if (wave < 2) add(sum[wave]);
+  if (wave == 1) put(sum[1]);   // read by this wavefront alone before
+  __syncthreads();
+  if (wave == 0) {
+    add(sum[1]);
+    put(partial + (size_t)blockIdx.x * (NT * 256));
+  }
 }
 
-// G(i0 + i, j0 + j) = sum over the nb partial blocks, in workgroup order
-__global__ __launch_bounds__(KS_BLOCK) void k_gram_fin(const double *__restrict__ partial, int nb, int qb, int pb,
-                                                      int i0, int j0, double *__restrict__ G, int ldg) {
-  const int e = blockIdx.x * KS_BLOCK + threadIdx.x;   // entry of the 64 x 64 block
-  if (e >= 4096) return;
-  const int i = e >> 6, j = e & 63;
+// G(i0 + i, j0 + j) = sum over the nb workgroups' blocks of nt tiles: 16 entries a
+// workgroup, 16 threads an entry each adding every 16th block, then those 16 in order
+__global__ __launch_bounds__(KS_BLOCK) void k_gram_fin(const double *__restrict__ partial, int nb, int nt, int nx, int sym,
+                                                      int qb, int pb, int i0, int j0, double *__restrict__ G, int ldg) {
+  __shared__ double part[16][17];
+  const int el = threadIdx.x & 15, sl = threadIdx.x >> 4, e = blockIdx.x * 16 + el;
   double s = 0.0;
-  for (int b = 0; b < nb; b++) s += partial[(size_t)b * 4096 + e];
-  if (i < qb && j < pb) G[(size_t)(i0 + i) + (size_t)(j0 + j) * ldg] = s;
+#pragma unroll 8
+  for (int b = sl; b < nb; b += 16) s += partial[(size_t)b * nt * 256 + e];
+  part[sl][el] = s;
+  __syncthreads();
+  if (sl) return;
+  s = 0.0;
+#pragma unroll
+  for (int k = 0; k < 16; k++) s += part[k][el];
+  // entry e: register (e / 64) % 4 of lane e % 64 of tile e / 256 (row l / 16 + 4 q, column l % 16)
+  const int t = e >> 8, l = e & 63;
+  int a, c;
+  if (sym) {
+    a = t >= 6 ? 3 : t >= 3 ? 2 : t >= 1 ? 1 : 0;
+    c = t - a * (a + 1) / 2;
+  } else {
+    a = t / nx;
+    c = t - a * nx;
+  }
+  const int i = 16 * a + (l >> 4) + 4 * ((e >> 6) & 3), j = 16 * c + (l & 15);
+  if (i < qb && j < pb) {
+    G[(size_t)(i0 + i) + (size_t)(j0 + j) * ldg] = s;
+    if (sym && a != c) G[(size_t)(i0 + j) + (size_t)(j0 + i) * ldg] = s;
+  }
+}
+
+template <typename T, int NY>
+void launch_gram(ks_ctx ctx, int nx, bool sym, int nb, const T *X, long ldx, int p, const T *Y, long ldy, int q, int n, int rpw,
+                 int i0, int j0) {
+#define KS_GRAM_L(NX, SY)                                                                                                  \
+  hipLaunchKernelGGL((k_gram<T, NY, NX, SY>), dim3(nb), dim3(KS_BLOCK), 0, ctx->stream, X, ldx, p, Y, ldy, q, n, rpw, i0, \
+                     j0, ctx->d_partial)
+  if (sym) KS_GRAM_L(NY, true);
+  else if (nx == 1) KS_GRAM_L(1, false);
+  else if (nx == 2) KS_GRAM_L(2, false);
+  else if (nx == 3) KS_GRAM_L(3, false);
+  else KS_GRAM_L(4, false);
+#undef KS_GRAM_L
 }
 
 template <typename T>
 int gram_t(ks_ctx ctx, int n, const T *X, long ldx, int p, const T *Y, long ldy, int q, double *Gdev, int ldg) {
-  int nb = 0, rpb = 0;   // n == 0: no partial blocks, the finisher writes zeros
+  // workgroups: at least two steps a wavefront, at most two workgroups a CU; n == 0: no partial blocks, the
+  // finisher writes zeros
+  int nb = 0, rpw = 0;
   if (n > 0) {
-    nb = (n + KS_GRAM_ROWS - 1) / KS_GRAM_ROWS;
+    const long per = 2L * KS_GRAM_ROWS * KS_WAVES;
+    nb = (int)((n + per - 1) / per);
     if (nb > KS_GRAM_MAXB) nb = KS_GRAM_MAXB;
-    rpb = ((n + nb - 1) / nb + KS_GRAM_ROWS - 1) / KS_GRAM_ROWS * KS_GRAM_ROWS;
-    nb = (n + rpb - 1) / rpb;
+    rpw = (int)(((long)n + nb * KS_WAVES - 1) / (nb * KS_WAVES) + KS_GRAM_ROWS - 1) / KS_GRAM_ROWS * KS_GRAM_ROWS;
+    nb = (int)(((long)n + (long)rpw * KS_WAVES - 1) / ((long)rpw * KS_WAVES));
   }
   static_assert((size_t)KS_GRAM_MAXB * 4096 <= (size_t)KS_MAXB * KS_NCOLP, "Gram partials exceed the workspace");
   for (int i0 = 0; i0 < q; i0 += 64)
     for (int j0 = 0; j0 < p; j0 += 64) {
-      if (nb > 0)
-        hipLaunchKernelGGL((k_gram<T>), dim3(nb), dim3(KS_BLOCK), 0, ctx->stream, X, ldx, p, Y, ldy, q, n, rpb, i0,
-                           j0, ctx->d_partial);
-      hipLaunchKernelGGL(k_gram_fin, dim3(4096 / KS_BLOCK), dim3(KS_BLOCK), 0, ctx->stream,
-                         (const double *)ctx->d_partial, nb, min(64, q - i0), min(64, p - j0), i0, j0, Gdev, ldg);
+      const int ny = (min(64, q - i0) + 15) / 16, nx = (min(64, p - j0) + 15) / 16;
+      const bool sym = i0 == j0 && p == q && (const void *)X == (const void *)Y && ldx == ldy;
+      const int nt = sym ? ny * (ny + 1) / 2 : ny * nx;
+      if (nb > 0) {
+        if (ny == 1) launch_gram<T, 1>(ctx, nx, sym, nb, X, ldx, p, Y, ldy, q, n, rpw, i0, j0);
+        else if (ny == 2) launch_gram<T, 2>(ctx, nx, sym, nb, X, ldx, p, Y, ldy, q, n, rpw, i0, j0);
+        else if (ny == 3) launch_gram<T, 3>(ctx, nx, sym, nb, X, ldx, p, Y, ldy, q, n, rpw, i0, j0);
+        else launch_gram<T, 4>(ctx, nx, sym, nb, X, ldx, p, Y, ldy, q, n, rpw, i0, j0);
+      }
+      hipLaunchKernelGGL(k_gram_fin, dim3(nt * 16), dim3(KS_BLOCK), 0, ctx->stream, (const double *)ctx->d_partial, nb, nt,
+                         nx, (int)sym, min(64, q - i0), min(64, p - j0), i0, j0, Gdev, ldg);
     }
   KS_HIP(hipGetLastError());
   return KS_OK;
