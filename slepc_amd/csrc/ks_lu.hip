@@ -235,142 +235,268 @@ __device__ inline void pub_wait(const unsigned long long *w, unsigned epoch, uns
   }
 }
 
-// The whole sub-panel in one cooperative launch (all G workgroups resident):
-// thread t of workgroup g keeps row j0 + g * KS_LU_PT + t of the 64 panel
-// columns in LDS for the 64 column steps, which exchange their data through
-// epoch-tagged words instead of launch boundaries.  Per column k (epoch
-// e0 + k): each workgroup finds its best candidate (largest magnitude, lowest
-// row) and publishes it -- its (magnitude, row) as three words, the row's
-// values in columns k..63 as two words each, one value a thread -- into slot
-// k & 1; every workgroup then waits for the G candidates, takes the best
-// (ties to the lower row), waits for the winner's values and updates its rows
-// as k_lu_step does (the same operations in the same order: the factors are
-// those of the column-step launches).  A workgroup writes slot k & 1 again
-// only at column k + 2, after every workgroup has published column k + 1,
-// which each does after reading column k.
+// keeps the better of a lane's candidate and lane ^ OFF's
+template <int OFF>
+__device__ __forceinline__ void piv_xor(double &m, int &i) {
+  double om;
+  int oi;
+  if constexpr (OFF >= 16) {
+    double a = __longlong_as_double((long long)i), b = a;
+    om = m;
+    ks_lane_swap<OFF>(m, om);
+    ks_lane_swap<OFF>(a, b);
+    i = (int)__double_as_longlong(a);
+    oi = (int)__double_as_longlong(b);
+  } else {
+    om = ks_lane_xor<OFF>(m);
+    oi = ks_lane_xor32<OFF>(i);
+  }
+  if (piv_better(om, oi, m, i)) {
+    m = om;
+    i = oi;
+  }
+}
+__device__ __forceinline__ void piv_wave(double &m, int &i) {
+  piv_xor<32>(m, i);
+  piv_xor<16>(m, i);
+  piv_xor<8>(m, i);
+  piv_xor<4>(m, i);
+  piv_xor<2>(m, i);
+  piv_xor<1>(m, i);
+}
+
+// The whole sub-panel in one launch (all G workgroups resident): thread t of
+// workgroup g keeps row j0 + g * KS_LU_PT + t of the 64 panel columns in LDS for
+// the 64 column steps, which exchange their data through epoch-tagged words
+// instead of launch boundaries.  Per column k (epoch e0 + k) each workgroup
+// publishes its best candidate (largest magnitude, lowest row) -- (magnitude,
+// row) as three words, the row's values in columns k..63 as two words each, one
+// value a thread -- in slot k & 1; every workgroup waits for the G candidates,
+// takes the best (ties to the lower row), waits for the winner's values and
+// updates its rows as k_lu_step does (the same operations in the same order: the
+// factors are those of the column-step launches).  Column k + 1 is updated first
+// and its candidate published before the other columns are, so that the update
+// and the candidates' way through the fabric overlap; a row's values follow.  A
+// workgroup writes slot k & 1 again only at column k + 2, after every workgroup has
+// published its candidate of column k + 1, which each does after reading column k.
+// Bound by the two exchanges of a column: PANEL_TABLE
 #define KS_LU_PT 128                                  // rows (threads) a workgroup
 #define KS_LU_PW (KS_LU_PT / 64)
 #define KS_LU_CO_MAX 256                              // workgroups at most (ldn <= 32,768)
+#define KS_LU_ORD_MAX 128                             // ... of an ordinary launch
 #define KS_LU_CAND 3                                  // words of a candidate: magnitude (2), row
 __global__ __launch_bounds__(KS_LU_PT) void k_lu_panel(double *__restrict__ A, int ldn, int j0,
                                                       unsigned long long *cand, unsigned long long *crow,
                                                       unsigned e0, int *__restrict__ prow, int *flag, int *err) {
   __shared__ double rowv[KS_LU_NB][KS_LU_PT];   // 64 KB: the workgroup's rows of the panel
-  __shared__ double pv[KS_LU_NB];
-  __shared__ double sm[KS_LU_PW];
-  __shared__ int si[KS_LU_PW];
-  __shared__ int s_best, s_p;
-  const int tid = threadIdx.x, G = gridDim.x, g = blockIdx.x;
-  const int r = j0 + g * KS_LU_PT + tid;
+  __shared__ __attribute__((aligned(16))) double pv[KS_LU_NB];
+  __shared__ double sm[2][KS_LU_PW];
+  __shared__ int si[2][KS_LU_PW];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, G = gridDim.x, g = blockIdx.x;
+  const int g0 = j0 + g * KS_LU_PT, r = g0 + tid;
   const bool have = r < ldn;
+  // the workgroup's best candidate, in every thread; which: two uses never share a slot between barriers
+  auto best = [&](double &m, int &i, int which) __attribute__((always_inline)) {
+    piv_wave(m, i);
+    if (lane == 0) {
+      sm[which][wave] = m;
+      si[which][wave] = i;
+    }
+    __syncthreads();
+    m = sm[which][0];
+    i = si[which][0];
+#pragma unroll
+    for (int w = 1; w < KS_LU_PW; w++)
+      if (piv_better(sm[which][w], si[which][w], m, i)) {
+        m = sm[which][w];
+        i = si[which][w];
+      }
+  };
+  // the candidate of column k
+  auto send_cand = [&](int k, double m, int i) __attribute__((always_inline)) {
+    if (tid == 0) {
+      unsigned long long *w = cand + ((size_t)(k & 1) * KS_LU_CO_MAX + g) * KS_LU_CAND;
+      pub_store_f64(w, e0 + (unsigned)k, m);
+      pub_store(w + 2, e0 + (unsigned)k, (unsigned)i);
+    }
+  };
+  // its values, columns k..63, one a thread (the row's index -> its thread)
+  auto send_row = [&](int k, int i) __attribute__((always_inline)) {
+    const int c = k + tid;
+    if (c < KS_LU_NB)
+      pub_store_f64(crow + ((size_t)(k & 1) * KS_LU_CO_MAX + g) * 2 * KS_LU_NB + 2 * c, e0 + (unsigned)k,
+                    i != INT_MAX ? rowv[c][i - g0] : 0.0);
+  };
 #pragma unroll 8
   for (int c = 0; c < KS_LU_NB; c++) rowv[c][tid] = have ? A[(size_t)r + (size_t)(j0 + c) * ldn] : 0.0;
   bool used = !have;
-  __syncthreads();
+  double m = used ? -1.0 : piv_mag(rowv[0][tid]);
+  int idx = used ? INT_MAX : r;
+  best(m, idx, 0);
+  send_cand(0, m, idx);
+  send_row(0, idx);
   for (int k = 0; k < KS_LU_NB; k++) {
     const unsigned ep = e0 + (unsigned)k;
     const int slot = k & 1;
-    unsigned long long *mycand = cand + ((size_t)slot * KS_LU_CO_MAX + g) * KS_LU_CAND;
-    unsigned long long *myrow = crow + ((size_t)slot * KS_LU_CO_MAX + g) * 2 * KS_LU_NB;
-    double m = used ? -1.0 : piv_mag(rowv[k][tid]);
-    int idx = used ? INT_MAX : r;
-    piv_reduce<KS_LU_PW>(m, idx, sm, si);
-    if (tid == 0) {
-      s_best = idx;
-      pub_store_f64(mycand, ep, m);
-      pub_store(mycand + 2, ep, (unsigned)idx);
-    }
-    __syncthreads();
-    {   // the candidate's values, columns k..63, one a thread (the row's index -> its thread)
-      const int b = s_best;
-      const int c = k + tid;
-      if (c < KS_LU_NB) pub_store_f64(myrow + 2 * c, ep, b != INT_MAX ? rowv[c][b - (j0 + g * KS_LU_PT)] : 0.0);
-    }
     // the best of the G candidates (each workgroup alike)
     double mb = -1.0;
-    int ib = INT_MAX;
+    int p = INT_MAX;
     for (int q = tid; q < G; q += KS_LU_PT) {
       unsigned w[KS_LU_CAND];
       pub_wait<KS_LU_CAND>(cand + ((size_t)slot * KS_LU_CO_MAX + q) * KS_LU_CAND, ep, w, err);
       const double a = __longlong_as_double((long long)(((unsigned long long)w[1] << 32) | w[0]));
       const int i = (int)w[2];
-      if (piv_better(a, i, mb, ib)) {
+      if (piv_better(a, i, mb, p)) {
         mb = a;
-        ib = i;
+        p = i;
       }
     }
-    piv_reduce<KS_LU_PW>(mb, ib, sm, si);
-    if (tid == 0) {
-      s_p = ib;
-      if (g == 0) {
-        prow[k] = ib;
-        if (!(mb >= KS_LU_ZEROPIVOT)) *flag = 1;
-      }
+    best(mb, p, 1);
+    if (tid == 0 && g == 0) {
+      prow[k] = p;
+      if (!(mb >= KS_LU_ZEROPIVOT)) *flag = 1;
     }
-    __syncthreads();
-    const int p = s_p;
-    const int gw = p == INT_MAX ? g : (p - j0) / KS_LU_PT;   // a candidate row always exists
+    const int gw = p < j0 || p >= ldn ? g : (p - j0) / KS_LU_PT;   // a candidate row always exists, unless a wait ran out
     if (tid >= k && tid < KS_LU_NB) {
       unsigned w[2];
       pub_wait<2>(crow + ((size_t)slot * KS_LU_CO_MAX + gw) * 2 * KS_LU_NB + 2 * tid, ep, w, err);
       pv[tid] = __longlong_as_double((long long)(((unsigned long long)w[1] << 32) | w[0]));
     }
     __syncthreads();
-    if (!used) {
-      if (r == p) {
-        used = true;
-      } else {
-        const double l = rowv[k][tid] * (1.0 / pv[k]);
-        rowv[k][tid] = l;
-        for (int c = k + 1; c < KS_LU_NB; c++) rowv[c][tid] -= l * pv[c];
+    double l = 0.0;
+    const bool upd = !used && r != p;
+    if (r == p) used = true;
+    if (upd) {
+      l = rowv[k][tid] * (1.0 / pv[k]);
+      rowv[k][tid] = l;
+    }
+    if (k + 1 == KS_LU_NB) break;
+    m = -1.0;
+    idx = INT_MAX;
+    if (upd) {
+      const double x = rowv[k + 1][tid] - l * pv[k + 1];
+      rowv[k + 1][tid] = x;
+      m = piv_mag(x);
+      idx = r;
+    }
+    best(m, idx, 0);
+    send_cand(k + 1, m, idx);
+    if (upd) {
+      for (int c = (k + 2) & ~7; c < KS_LU_NB; c += 8) {
+        double x[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) x[u] = rowv[c + u][tid];
+#pragma unroll
+        for (int u = 0; u < 8; u++) x[u] = c + u >= k + 2 ? x[u] - l * pv[c + u] : x[u];
+#pragma unroll
+        for (int u = 0; u < 8; u++) rowv[c + u][tid] = x[u];
       }
     }
     __syncthreads();
+    send_row(k + 1, idx);
   }
 #pragma unroll 8
   for (int c = 0; c < KS_LU_NB; c++)
     if (have) A[(size_t)r + (size_t)(j0 + c) * ldn] = rowv[c][tid];
 }
 
-// the pivot rows of the panel (physical rows, chosen in place) as LAPACK's
+// the pivot rows of the sub-panel (physical rows, chosen in place) as LAPACK's
 // interchanges: at step j rows j and ipiv[j] swap.  Only rows that started in
-// the panel's own 64 positions can sit elsewhere when picked: lpos follows
-// where those rows are, at which of the 64 positions holds which row.
-__global__ __launch_bounds__(64) void k_lu_ipiv(const int *__restrict__ prow, int j0, int *__restrict__ ipiv) {
-  __shared__ int lpos[KS_LU_NB], at[KS_LU_NB];
-  lpos[threadIdx.x] = j0 + threadIdx.x;
-  at[threadIdx.x] = j0 + threadIdx.x;
+// the sub-panel's own 64 positions can sit elsewhere when picked: lpos follows
+// where those rows are, at which of the 64 positions holds which row.  What the
+// interchanges do together is a move of at most 128 rows, row src[i] to row
+// dst[i] (dst -1: none): the picked rows to the 64 positions, the rows that stood
+// there and were not picked to where the picked ones were.  cur follows the rows
+// over the sub-panels of a panel.
+__global__ __launch_bounds__(64) void k_lu_ipiv(const int *__restrict__ prow, int j0, int ldn, int *__restrict__ ipiv,
+                                               int *__restrict__ cur, int *__restrict__ dst, int *__restrict__ src) {
+  __shared__ int lpos[KS_LU_NB], at[KS_LU_NB], pr[KS_LU_NB], ip[KS_LU_NB];
+  const int t = threadIdx.x;
+  lpos[t] = j0 + t;
+  at[t] = j0 + t;
+  pr[t] = prow[t] >= j0 && prow[t] < ldn ? prow[t] : j0 + t;   // out of range only after a wait that ran out
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (t == 0) {
     for (int k = 0; k < KS_LU_NB; k++) {
-      const int j = j0 + k, p = prow[k];
+      const int j = j0 + k, p = pr[k];
       const bool pin = p - j0 < KS_LU_NB;
       const int P = pin ? lpos[p - j0] : p;   // where row p stands now (>= j)
-      ipiv[j] = P;
-      const int x = at[k];                    // the row standing at j, one of the panel's own
+      ip[k] = P;
+      const int x = at[k];                    // the row standing at j, one of the sub-panel's own
       lpos[x - j0] = P;
       if (pin) lpos[p - j0] = j;
       at[k] = p;
       if (P - j0 < KS_LU_NB) at[P - j0] = x;
     }
   }
+  __syncthreads();
+  ipiv[j0 + t] = ip[t];
+  const int s0 = pr[t], d1 = lpos[t] >= j0 + KS_LU_NB ? lpos[t] : -1;
+  dst[t] = j0 + t;
+  src[t] = s0;
+  dst[KS_LU_NB + t] = d1;
+  src[KS_LU_NB + t] = j0 + t;
+  const int c0 = cur[s0], c1 = cur[j0 + t];
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // every lane has read before one writes
+  __syncthreads();
+  cur[j0 + t] = c0;
+  if (d1 >= 0) cur[d1] = c1;
 }
 
-// the panel's interchanges (rows j0..j0+NB-1 with ipiv, in order) on the columns
-// cb .. cb+nc-1, a thread per column
-__global__ __launch_bounds__(KS_BLOCK) void k_lu_laswp(double *__restrict__ A, int ldn, int j0,
-                                                      const int *__restrict__ ipiv, int cb, int nc) {
-  const int t = blockIdx.x * KS_BLOCK + threadIdx.x;
-  if (t >= nc) return;
-  double *a = A + (size_t)(cb + t) * ldn;
-  for (int j = j0; j < j0 + KS_LU_NB; j++) {
-    const int p = ipiv[j];
-    if (p != j) {
-      const double x = a[j];
-      a[j] = a[p];
-      a[p] = x;
+// the moves of a whole panel (its columns from J0): the rows cur has elsewhere, at
+// most twice the panel's columns; cur is the identity again
+__global__ __launch_bounds__(1024) void k_lu_moves(int *__restrict__ cur, int J0, int ldn, int *__restrict__ dst,
+                                                  int *__restrict__ src, int *__restrict__ cnt) {
+  __shared__ int m;
+  if (threadIdx.x == 0) m = 0;
+  __syncthreads();
+  for (int i = J0 + threadIdx.x; i < ldn; i += 1024) {
+    const int c = cur[i];
+    if (c != i) {
+      const int e = atomicAdd(&m, 1);
+      if (e < 2 * KS_LU_NB2) {
+        dst[e] = i;
+        src[e] = c;
+      }
+      cur[i] = i;
     }
   }
+  __syncthreads();
+  if (threadIdx.x == 0) *cnt = min(m, 2 * KS_LU_NB2);
+}
+
+// Row moves on the columns outside [skip, skip + nskip) of cb .. cb+nc-1, a wavefront a
+// column: all (*cnt, or PL * 64) values are read, then written.  A sub-panel's
+// (PL = 2) go to its panel's columns only, and the other columns take the panel's
+// (PL = 16) at once, where consecutive rows share cache lines: for n = 16,256 this was
+// 29 ms as interchanges of every sub-panel on all columns by a thread a column.
+template <int PL>
+__global__ __launch_bounds__(KS_BLOCK) void k_lu_move(double *__restrict__ A, int ldn, const int *__restrict__ dst,
+                                                     const int *__restrict__ src, const int *__restrict__ cnt, int cb,
+                                                     int nc, int skip, int nskip) {
+  const int lane = threadIdx.x & 63;
+  int c = cb + blockIdx.x * KS_WAVES + (threadIdx.x >> 6);
+  if (c >= cb + nc - nskip) return;
+  if (c >= skip) c += nskip;
+  double *a = A + (size_t)c * ldn;
+  const int m = cnt ? *cnt : 64 * PL;
+  int d[PL];
+  double v[PL];
+#pragma unroll
+  for (int u = 0; u < PL; u++) {
+    const int e = lane + 64 * u;
+    d[u] = e < m ? dst[e] : -1;
+    v[u] = d[u] >= 0 ? a[src[e]] : 0.0;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the wavefront's reads before its writes
+#pragma unroll
+  for (int u = 0; u < PL; u++)
+    if (d[u] >= 0) a[d[u]] = v[u];
+}
+
+__global__ __launch_bounds__(KS_BLOCK) void k_lu_iota(int *__restrict__ cur, int n) {
+  const int i = blockIdx.x * KS_BLOCK + threadIdx.x;
+  if (i < n) cur[i] = i;
 }
 
 // U12 = L11^-1 A12 for the columns cb .. cb+ncols-1: a wavefront per column,
@@ -633,9 +759,10 @@ int lu_factor(ks_ctx ctx, ks_csr A, double sigma, ks_lu *out, bool coop) {
   const int n = A->nrows, ldn = (n + KS_LU_NB - 1) / KS_LU_NB * KS_LU_NB;
   F->n = n;
   F->ldn = ldn;
-  // factorization scratch: used[ldn], prow[64], flag, err, pi[2][PG_MAX] (ints); pm[2][PG_MAX]
+  // factorization scratch: used[ldn], prow[64], flag, err, pi[2][PG_MAX], cur[ldn], the row moves' count,
+  // dst[128], src[128] of a sub-panel and dst[1024], src[1024] of a panel (ints); pm[2][PG_MAX]
   // (doubles); the cooperative panels' published words cand[2][CO_MAX][3], crow[2][CO_MAX][2 * 64]
-  const size_t nint = (size_t)ldn + KS_LU_NB + 2 + 2 * KS_LU_PG_MAX;
+  const size_t nint = 2 * (size_t)ldn + KS_LU_NB + 3 + 2 * KS_LU_PG_MAX + 4 * (KS_LU_NB + KS_LU_NB2);
   const size_t off_dbl = ((nint * sizeof(int) + 255) / 256) * 256;
   const size_t nwords = 2 * KS_LU_CO_MAX * (KS_LU_CAND + 2 * KS_LU_NB);
   const size_t scratch_bytes = off_dbl + 2 * KS_LU_PG_MAX * sizeof(double) + nwords * sizeof(unsigned long long);
@@ -659,6 +786,8 @@ int lu_factor(ks_ctx ctx, ks_csr A, double sigma, ks_lu *out, bool coop) {
   }
   int *d_used = (int *)scratch, *d_prow = d_used + ldn, *d_flag = d_prow + KS_LU_NB, *d_perr = d_flag + 1,
       *d_pi = d_perr + 1;
+  int *d_cur = d_pi + 2 * KS_LU_PG_MAX, *d_cnt = d_cur + ldn, *d_dst = d_cnt + 1, *d_src = d_dst + 2 * KS_LU_NB,
+      *d_pdst = d_src + 2 * KS_LU_NB, *d_psrc = d_pdst + 2 * KS_LU_NB2;
   double *d_pm = (double *)((char *)scratch + off_dbl);
   unsigned long long *d_cand = (unsigned long long *)(d_pm + 2 * KS_LU_PG_MAX);
   unsigned long long *d_crow = d_cand + 2 * KS_LU_CO_MAX * KS_LU_CAND;
@@ -668,6 +797,8 @@ int lu_factor(ks_ctx ctx, ks_csr A, double sigma, ks_lu *out, bool coop) {
   const int fill_blocks = (ldn + KS_BLOCK - 1) / KS_BLOCK;
   hipLaunchKernelGGL(k_lu_fill, dim3(fill_blocks), dim3(KS_BLOCK), 0, st, A->d_rowptr, A->d_colidx,
                      (const double *)A->d_val, n, ldn, sigma, F->d_A);
+  hipLaunchKernelGGL(k_lu_iota, dim3(fill_blocks), dim3(KS_BLOCK), 0, st, d_cur, ldn);
+  auto move_blocks = [](int nc) { return dim3((nc + KS_WAVES - 1) / KS_WAVES); };
   // panels of KS_LU_NB2 columns, each factored as sub-panels of KS_LU_NB (dgetrf2's
   // recursion cut at 64): a sub-panel is first brought up to date with the earlier
   // sub-panels of its panel, and the columns right of the panel take the whole
@@ -701,9 +832,17 @@ int lu_factor(ks_ctx ctx, ks_csr A, double sigma, ks_lu *out, bool coop) {
         unsigned a_e0 = e0;
         int *a_prow = d_prow, *a_flag = d_flag, *a_err = d_perr;
         void *args[] = {&a_A, &a_ldn, &a_j0, &a_cand, &a_crow, &a_e0, &a_prow, &a_flag, &a_err};
-        if (hipLaunchCooperativeKernel((const void *)k_lu_panel, dim3(Gc), dim3(KS_LU_PT), args, 0, st) ==
-            hipSuccess)
-          e0 += KS_LU_NB;
+        // Up to KS_LU_ORD_MAX workgroups, two of which fit a CU, one launch of each of the four
+        // hardware queues HIP uses fits the chip, and an ordinary launch does (a wait that runs out
+        // all the same is seen below); more go out as a cooperative launch, which waits for the
+        // queue to drain first: LU_COOP
+        bool sent = Gc <= KS_LU_ORD_MAX;
+        if (sent)
+          hipLaunchKernelGGL(k_lu_panel, dim3(Gc), dim3(KS_LU_PT), 0, st, F->d_A, ldn, j0, d_cand, d_crow, e0, d_prow, d_flag,
+                             d_perr);
+        else
+          sent = hipLaunchCooperativeKernel((const void *)k_lu_panel, dim3(Gc), dim3(KS_LU_PT), args, 0, st) == hipSuccess;
+        if (sent) e0 += KS_LU_NB;
         else {
           (void)hipGetLastError();
           coop = false;
@@ -717,9 +856,14 @@ int lu_factor(ks_ctx ctx, ks_csr A, double sigma, ks_lu *out, bool coop) {
           hipLaunchKernelGGL(k_lu_step, dim3(G), dim3(KS_BLOCK), 0, st, F->d_A, ldn, j0, j, d_used, d_pm, d_pi,
                              d_prow, d_flag);
       }
-      hipLaunchKernelGGL(k_lu_ipiv, dim3(1), dim3(KS_LU_NB), 0, st, (const int *)d_prow, j0, F->d_ipiv);
-      hipLaunchKernelGGL(k_lu_laswp, dim3(fill_blocks), dim3(KS_BLOCK), 0, st, F->d_A, ldn, j0,
-                         (const int *)F->d_ipiv, 0, ldn);
+      hipLaunchKernelGGL(k_lu_ipiv, dim3(1), dim3(KS_LU_NB), 0, st, (const int *)d_prow, j0, ldn, F->d_ipiv, d_cur, d_dst, d_src);
+      hipLaunchKernelGGL(k_lu_move<2>, move_blocks(W), dim3(KS_BLOCK), 0, st, F->d_A, ldn, (const int *)d_dst,
+                         (const int *)d_src, (const int *)nullptr, J0, W, J0 + W, 0);
+    }
+    if (ldn > W) {
+      hipLaunchKernelGGL(k_lu_moves, dim3(1), dim3(1024), 0, st, d_cur, J0, ldn, d_pdst, d_psrc, d_cnt);
+      hipLaunchKernelGGL(k_lu_move<2 * KS_LU_NB2 / 64>, move_blocks(ldn - W), dim3(KS_BLOCK), 0, st, F->d_A, ldn,
+                         (const int *)d_pdst, (const int *)d_psrc, (const int *)d_cnt, 0, ldn, J0, W);
     }
     const int cb = J0 + W, nc = ldn - cb;
     if (nc > 0) {   // U12 of the panel's rows, then A22 -= L21 U12 with K = W
