@@ -5,8 +5,8 @@
 // Reductions are row-partitioned: each workgroup owns RPT*256 consecutive rows,
 // keeps its slice of the vector in registers, sweeps the columns in tiles of
 // KS_CT, reduces each tile across its four wavefronts (DPP/shuffle + LDS) and
-// writes one partial row; the last workgroup of each group of 32 and then the
-// last group finish the sums in a fixed order (deterministic, no float atomics).
+// writes one partial row; a second launch adds the rows in a fixed order
+// (deterministic, no float atomics).
 #include "ks_internal.hpp"
 
 #include <cmath>
@@ -17,31 +17,16 @@
 
 namespace {
 
-enum { GS_FIRST = 0, GS_REPEAT = 1, GS_PLAIN = 2 };
-
 template <typename T> struct acc_t { using type = double; };
 template <> struct acc_t<float> { using type = float; };
 
-__device__ __forceinline__ bool gs_gate(const ks_status *st, int mode, int col, int pass) {
-  if (mode == GS_FIRST) return st->active != 0;
-  if (mode == GS_REPEAT) return st->active && st->col == col && !st->done && st->pass_done == pass - 1;
-  return true;
-}
-
-// partial[b][0..ntot) = V(rows_b, 0..k)^T w(rows_b)  (+ w^T w at column k unless PLAIN)
-template <typename T, int RPT, int MODE>
-__global__ __launch_bounds__(KS_BLOCK) void k_gs_dot(const T *__restrict__ V, long ld, int k,
-                                                    const T *__restrict__ w, int n, int nblocks,
-                                                    double *partial, double *gpartial, unsigned *counters,
-                                                    ks_status *st, double *cout, double *hcol, int col,
-                                                    int pass, int *ran, double deftol) {
+// partial[b][0..k) = V(rows_b, 0..k)^T w(rows_b)
+template <typename T, int RPT>
+__global__ __launch_bounds__(KS_BLOCK) void k_dot(const T *__restrict__ V, long ld, int k, const T *__restrict__ w, int n,
+                                                 double *__restrict__ partial) {
   using AT = typename acc_t<T>::type;
-  if (MODE != GS_PLAIN && !gs_gate(st, MODE, col, pass)) return;
-  if (ran && blockIdx.x == 0 && threadIdx.x == 0) *ran = 1;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int ntot = MODE == GS_PLAIN ? k : k + 1;
   __shared__ double sh[KS_WAVES * KS_CT];
-  __shared__ double fin[KS_NCOLP];
   const size_t row0 = (size_t)blockIdx.x * KS_BLOCK * RPT;
   T wv[RPT];
   bool ok[RPT];
@@ -51,7 +36,7 @@ __global__ __launch_bounds__(KS_BLOCK) void k_gs_dot(const T *__restrict__ V, lo
     ok[r] = i < (size_t)n;
     wv[r] = ok[r] ? w[i] : (T)0;
   }
-  for (int c0 = 0; c0 < ntot; c0 += KS_CT) {
+  for (int c0 = 0; c0 < k; c0 += KS_CT) {
     AT acc[KS_CT];
 #pragma unroll
     for (int t = 0; t < KS_CT; t++) acc[t] = 0;
@@ -65,79 +50,54 @@ __global__ __launch_bounds__(KS_BLOCK) void k_gs_dot(const T *__restrict__ V, lo
         if (c < k) acc[t] += (AT)V[i + (size_t)c * ld] * (AT)wv[r];
       }
     }
-    double self = 0.0;
-    if (MODE != GS_PLAIN && c0 + KS_CT > k) {   // this tile holds the self dot (w^T w, FP64)
-#pragma unroll
-      for (int r = 0; r < RPT; r++) self += (double)wv[r] * (double)wv[r];
-    }
     // reduce the tile across the workgroup
 #pragma unroll
     for (int t = 0; t < KS_CT; t++) {
-      double v = (MODE != GS_PLAIN && c0 + t == k) ? self : (double)acc[t];
-      v = ks_wave_sum(v);
+      const double v = ks_wave_sum((double)acc[t]);
       if (lane == 0) sh[wave * KS_CT + t] = v;
     }
     __syncthreads();
-    if (tid < KS_CT && c0 + tid < ntot) {
+    if (tid < KS_CT && c0 + tid < k) {
       double s = 0.0;
 #pragma unroll
       for (int q = 0; q < KS_WAVES; q++) s += sh[q * KS_CT + tid];
-      partial[(size_t)blockIdx.x * ntot + c0 + tid] = s;
+      partial[(size_t)blockIdx.x * k + c0 + tid] = s;
     }
     __syncthreads();
-  }
-  if (!ks_reduce_finish(partial, gpartial, counters, nblocks, ntot, fin)) return;
-  // finishing workgroup.  With constraints the accumulated column may be the
-  // scratch column itself (column 0), so it is cleaned before c is written.
-  if (MODE == GS_FIRST) {
-    for (int c = tid; c <= k; c += KS_BLOCK) hcol[c] = 0.0;   // BV_CleanCoefficients
-    __syncthreads();
-  }
-  for (int c = tid; c < k; c += KS_BLOCK) cout[c] = fin[c];
-  if (MODE == GS_PLAIN) return;
-  if (tid == 0) {
-    const double self = fin[k];
-    double sumsq = 0.0;
-    for (int c = 0; c < k; c++) sumsq += fin[c] * fin[c];    // BV_SquareSum
-    st->sumsq = sumsq;
-    if (self < -deftol) {                                    // BV_SafeSqrt
-      st->error = KS_ERR_INNER;
-      st->active = 0;
-    }
-    st->onrm = self < 0.0 ? 0.0 : sqrt(self);
-    if (MODE == GS_FIRST) {
-      st->col = col;
-      st->pass_done = 0;
-      st->done = 0;
-      st->lindep = 0;
-    }
   }
 }
 
-// GS: w -= V(:,0..k) c, partial |w|^2, DGKS decision in the finishing workgroup.
-// PLAIN: w = beta*w + alpha*V c (no reduction).
-template <typename T, int RPT, int MODE>
-__global__ __launch_bounds__(KS_BLOCK) void k_gs_update(const T *__restrict__ V, long ld, int k, T *__restrict__ w,
-                                                       int n, int nblocks, const double *__restrict__ cin,
-                                                       double alpha, double beta, double *partial,
-                                                       double *gpartial, unsigned *counters, ks_status *st,
-                                                       double *hcol, int col, int pass, int refine, double eta,
-                                                       int do_scale, int safe, int *ran) {
-  using AT = typename acc_t<T>::type;
-  if (MODE == GS_FIRST) {
-    if (!(st->active && st->col == col && st->pass_done == 0 && !st->done)) return;
-  } else if (MODE == GS_REPEAT) {
-    if (!gs_gate(st, MODE, col, pass)) return;
+// cout[c] = the sum of the nb workgroups' partial[b][c], 16 columns a
+// workgroup, 16 threads a column each adding every 16th block, then those 16 in order.
+// A finish by k_dot's last workgroups behind fences and tickets cost more than this launch:
+// 22,500 rows, 10 columns 27 us in one launch against 8 + 5 in two.
+__global__ __launch_bounds__(KS_BLOCK) void k_dot_fin(const double *__restrict__ partial, int nb, int k, double *__restrict__ cout) {
+  __shared__ double part[16][17];
+  const int el = threadIdx.x & 15, sl = threadIdx.x >> 4, c = blockIdx.x * 16 + el;
+  double s = 0.0;
+  if (c < k) {
+#pragma unroll 8
+    for (int b = sl; b < nb; b += 16) s += partial[(size_t)b * k + c];
   }
-  if (ran && blockIdx.x == 0 && threadIdx.x == 0) *ran = 1;
+  part[sl][el] = s;
+  __syncthreads();
+  if (sl || c >= k) return;
+  s = 0.0;
+#pragma unroll
+  for (int q = 0; q < 16; q++) s += part[q][el];
+  cout[c] = s;
+}
+
+// w = beta w + alpha V c
+template <typename T, int RPT>
+__global__ __launch_bounds__(KS_BLOCK) void k_multvec(const T *__restrict__ V, long ld, int k, T *__restrict__ w, int n,
+                                                     const double *__restrict__ cin, double alpha, double beta) {
+  using AT = typename acc_t<T>::type;
   const int tid = threadIdx.x;
   __shared__ AT sc[KS_MAX_COLS];
-  __shared__ double red[KS_WAVES];
-  __shared__ double fin[2];
-  for (int c = tid; c < k; c += KS_BLOCK) sc[c] = (AT)(MODE == GS_PLAIN ? alpha * cin[c] : cin[c]);
+  for (int c = tid; c < k; c += KS_BLOCK) sc[c] = (AT)(alpha * cin[c]);
   __syncthreads();
   const size_t row0 = (size_t)blockIdx.x * KS_BLOCK * RPT;
-  double sq = 0.0;
 #pragma unroll
   for (int r = 0; r < RPT; r++) {
     const size_t i = row0 + (size_t)r * KS_BLOCK + tid;
@@ -152,54 +112,7 @@ __global__ __launch_bounds__(KS_BLOCK) void k_gs_update(const T *__restrict__ V,
     }
     for (; c < k; c++) a0 += (AT)V[i + (size_t)c * ld] * sc[c];
     const AT dot = (a0 + a1) + (a2 + a3);
-    AT res;
-    if (MODE == GS_PLAIN) res = (beta == 0.0 ? (AT)0 : (AT)beta * (AT)w[i]) + dot;
-    else res = (AT)w[i] - dot;
-    w[i] = (T)res;
-    sq += (double)res * (double)res;
-  }
-  if (MODE == GS_PLAIN) return;
-  double bs = ks_block_sum(sq, red);
-  if (tid == 0) partial[blockIdx.x] = bs;
-  if (!ks_reduce_finish(partial, gpartial, counters, nblocks, 1, fin)) return;
-  for (int c = tid; c < k; c += KS_BLOCK) hcol[c] += cin[c];   // BV_AddCoefficients
-  if (tid == 0) {
-    const double exact = sqrt(fin[0]);
-    st->exact_sq = fin[0];
-    st->total_passes += 1;
-    const int l = ++st->pass_done;
-    const double onrm = st->onrm;
-    double nrm = 0.0;
-    int lindep = 0, finalize = 1, have_norm = 1;
-    if (safe) {                                    // BV_OrthogonalizeColumn_Safe
-      lindep = 1;
-      have_norm = 0;
-    } else if (refine == KS_REFINE_NEVER) {
-      nrm = exact;
-      lindep = !(nrm != 0.0);
-    } else {
-      if (refine == KS_REFINE_ALWAYS && l < 2) {
-        finalize = 0;
-      } else {
-        nrm = onrm * onrm - st->sumsq;             // estimate |v'| from |v|
-        nrm = (nrm <= 0.0) ? exact : sqrt(nrm);
-        if (refine == KS_REFINE_IFNEEDED && l < 3 && nrm != 0.0 && fabs(nrm) < eta * fabs(onrm)) finalize = 0;
-        else lindep = !(nrm != 0.0 && fabs(nrm) >= eta * fabs(onrm));
-      }
-      st->nrm = nrm;
-    }
-    if (finalize) {
-      st->done = 1;
-      st->lindep = lindep;
-      st->nrm = nrm;
-      st->beta_last = nrm;
-      if (have_norm) hcol[k] = lindep ? 0.0 : nrm;   // BV_SetValue
-      st->scale = (do_scale && nrm != 1.0 && nrm != 0.0) ? 1.0 / nrm : 1.0;
-      if (lindep) {
-        st->active = 0;
-        st->breakdown_col = col;
-      }
-    }
+    w[i] = (T)((beta == 0.0 ? (AT)0 : (AT)beta * (AT)w[i]) + dot);
   }
 }
 
@@ -1484,32 +1397,21 @@ inline int ew_blocks(int n) {
   return b;
 }
 
-template <typename T, int MODE>
-void launch_dot(ks_ctx ctx, int rpt, int nb, const T *V, long ld, int k, const T *w, int n, double *cout,
-                double *hcol, int col, int pass, int *ran) {
+template <typename T>
+void launch_dot(ks_ctx ctx, int rpt, int nb, const T *V, long ld, int k, const T *w, int n, double *cout) {
   dim3 grid(nb), block(KS_BLOCK);
-  const double deftol = 10.0 * 2.220446049250313e-16;
-#define KS_DOT_CASE(R)                                                                                   \
-  case R:                                                                                                \
-    hipLaunchKernelGGL((k_gs_dot<T, R, MODE>), grid, block, 0, ctx->stream, V, ld, k, w, n, nb,          \
-                       ctx->d_partial, ctx->d_gpartial, ctx->d_counters, ctx->d_status, cout, hcol, col, \
-                       pass, ran, deftol);                                                               \
-    break;
+#define KS_DOT_CASE(R)                                                                                        \
+  case R: hipLaunchKernelGGL((k_dot<T, R>), grid, block, 0, ctx->stream, V, ld, k, w, n, ctx->d_partial); break;
   switch (rpt) { KS_DOT_CASE(1) KS_DOT_CASE(2) KS_DOT_CASE(4) KS_DOT_CASE(8) KS_DOT_CASE(16) }
 #undef KS_DOT_CASE
+  hipLaunchKernelGGL(k_dot_fin, dim3((k + 15) / 16), block, 0, ctx->stream, (const double *)ctx->d_partial, nb, k, cout);
 }
-
-template <typename T, int MODE>
-void launch_upd(ks_ctx ctx, int rpt, int nb, const T *V, long ld, int k, T *w, int n, const double *cin,
-                double alpha, double beta, double *hcol, int col, int pass, int refine, double eta, int do_scale,
-                int safe, int *ran) {
+template <typename T>
+void launch_multvec(ks_ctx ctx, int rpt, int nb, const T *V, long ld, int k, T *w, int n, const double *cin, double alpha,
+                    double beta) {
   dim3 grid(nb), block(KS_BLOCK);
-#define KS_UPD_CASE(R)                                                                                      \
-  case R:                                                                                                   \
-    hipLaunchKernelGGL((k_gs_update<T, R, MODE>), grid, block, 0, ctx->stream, V, ld, k, w, n, nb, cin,     \
-                       alpha, beta, ctx->d_partial, ctx->d_gpartial, ctx->d_counters, ctx->d_status, hcol,  \
-                       col, pass, refine, eta, do_scale, safe, ran);                                        \
-    break;
+#define KS_UPD_CASE(R)                                                                                                 \
+  case R: hipLaunchKernelGGL((k_multvec<T, R>), grid, block, 0, ctx->stream, V, ld, k, w, n, cin, alpha, beta); break;
   switch (rpt) { KS_UPD_CASE(1) KS_UPD_CASE(2) KS_UPD_CASE(4) KS_UPD_CASE(8) KS_UPD_CASE(16) }
 #undef KS_UPD_CASE
 }
@@ -1928,11 +1830,9 @@ int ks_bv_dotvec(ks_ctx ctx, ks_prec prec, int n, const void *V, int ld, int k, 
   const double s = prec == KS_F64 ? 8.0 : 4.0;
   ks_prof_begin(ctx, KS_PROF_DOTVEC, (k + 1.0) * n * s, 2.0 * k * n, false);
   if (prec == KS_F64)
-    launch_dot<double, GS_PLAIN>(ctx, rpt, nb, (const double *)V, ld, k, (const double *)y, n, d_q, nullptr, 0, 0,
-                                 nullptr);
+    launch_dot<double>(ctx, rpt, nb, (const double *)V, ld, k, (const double *)y, n, d_q);
   else
-    launch_dot<float, GS_PLAIN>(ctx, rpt, nb, (const float *)V, ld, k, (const float *)y, n, d_q, nullptr, 0, 0,
-                                nullptr);
+    launch_dot<float>(ctx, rpt, nb, (const float *)V, ld, k, (const float *)y, n, d_q);
   ks_prof_end(ctx);
   KS_HIP(hipGetLastError());
   return KS_OK;
@@ -1947,11 +1847,9 @@ int ks_bv_multvec(ks_ctx ctx, ks_prec prec, int n, double alpha, const void *V, 
   const double s = prec == KS_F64 ? 8.0 : 4.0;
   ks_prof_begin(ctx, KS_PROF_MULTVEC, (k + 2.0) * n * s, 2.0 * k * n, false);
   if (prec == KS_F64)
-    launch_upd<double, GS_PLAIN>(ctx, rpt, nb, (const double *)V, ld, k, (double *)y, n, d_q, alpha, beta, nullptr,
-                                 0, 0, 0, 0.0, 0, 0, nullptr);
+    launch_multvec<double>(ctx, rpt, nb, (const double *)V, ld, k, (double *)y, n, d_q, alpha, beta);
   else
-    launch_upd<float, GS_PLAIN>(ctx, rpt, nb, (const float *)V, ld, k, (float *)y, n, d_q, alpha, beta, nullptr, 0,
-                                0, 0, 0.0, 0, 0, nullptr);
+    launch_multvec<float>(ctx, rpt, nb, (const float *)V, ld, k, (float *)y, n, d_q, alpha, beta);
   ks_prof_end(ctx);
   KS_HIP(hipGetLastError());
   return KS_OK;

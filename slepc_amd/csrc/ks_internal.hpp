@@ -407,47 +407,6 @@ __device__ __forceinline__ double ks_block_sum(double v, double *sh) {
   return s;
 }
 
-// Two-level "last block finishes" reduction of per-block partial rows.
-// Every block has written partial[blockIdx.x * ncol + c] for c < ncol.  Returns
-// true in exactly one block, whose threads then find the totals in out[0..ncol)
-// (shared memory).  Summation order is fixed, so results are deterministic.
-// Counters are returned to zero by the finishing blocks.
-__device__ __forceinline__ bool ks_reduce_finish(double *partial, double *gpartial,
-                                                 unsigned *counters, int nblocks, int ncol,
-                                                 double *out) {
-  __shared__ unsigned s_ticket;
-  const int g = blockIdx.x / KS_GROUP;
-  const int gbeg = g * KS_GROUP;
-  const int gend = min(nblocks, gbeg + KS_GROUP);
-  const int ngroups = (nblocks + KS_GROUP - 1) / KS_GROUP;
-  __threadfence();
-  __syncthreads();
-  if (threadIdx.x == 0) s_ticket = atomicAdd(&counters[g], 1u);
-  __syncthreads();
-  if (s_ticket != (unsigned)(gend - gbeg - 1)) return false;
-  __threadfence();
-  for (int c = threadIdx.x; c < ncol; c += blockDim.x) {
-    double s = 0.0;
-    for (int b = gbeg; b < gend; b++) s += __builtin_nontemporal_load(&partial[(size_t)b * ncol + c]);
-    gpartial[(size_t)g * ncol + c] = s;
-  }
-  if (threadIdx.x == 0) counters[g] = 0u;
-  __threadfence();
-  __syncthreads();
-  if (threadIdx.x == 0) s_ticket = atomicAdd(&counters[KS_MAXG], 1u);
-  __syncthreads();
-  if (s_ticket != (unsigned)(ngroups - 1)) return false;
-  __threadfence();
-  for (int c = threadIdx.x; c < ncol; c += blockDim.x) {
-    double s = 0.0;
-    for (int q = 0; q < ngroups; q++) s += __builtin_nontemporal_load(&gpartial[(size_t)q * ncol + c]);
-    out[c] = s;
-  }
-  if (threadIdx.x == 0) counters[KS_MAXG] = 0u;
-  __syncthreads();
-  return true;
-}
-
 // rows per thread (1,2,4,8,16) and block count for a row-partitioned reduction
 inline void ks_rows_split(int n, int *rpt, int *nblocks) {
   int r = 1;
