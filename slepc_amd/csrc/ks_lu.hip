@@ -8,18 +8,18 @@
 // factored by the right-looking blocked algorithm of LAPACK's dgetrf: panels
 // of 512 columns, each factored as sub-panels of 64 (dgetrf2's recursion cut
 // at 64 columns), the columns right of a panel updated once per panel:
-//   * sub-panel: one cooperative launch (k_lu_panel), the 64 column steps
-//     exchanging candidates through epoch-tagged words; or, should that launch
-//     be refused or a wait run out, one launch per column (k_lu_step) -- the
+//   * sub-panel: one launch (k_lu_panel; cooperative above 128 workgroups), the
+//     64 column steps exchanging candidates through epoch-tagged words; or, should
+//     that launch be refused or a wait run out, one launch per column (k_lu_step) -- the
 //     same operations in the same order.  The pivot rows are found and used in
 //     place (implicit pivoting): per column the best candidate over all rows
 //     (largest magnitude, lowest row on ties) is the pivot, the other rows'
 //     entries of column j are scaled by its reciprocal and their sub-panel
 //     columns right of j updated (dgetf2's dscal and dger).  Rows already
-//     chosen as pivots are skipped.  At the sub-panel's end one thread turns the pivot rows into
-//     LAPACK's sequence of interchanges, which are then applied to every
-//     column (dlaswp) -- the same rows and values dgetf2 arrives at by
-//     swapping as it goes;
+//     chosen as pivots are skipped.  At the sub-panel's end one thread turns the pivot
+//     rows into LAPACK's sequence of interchanges (dlaswp) -- the same rows and values
+//     dgetf2 arrives at by swapping as it goes -- and the rows they move are moved
+//     on the panel's columns; the columns outside take a panel's moves at once;
 //   * U12 = L11^-1 A12 per 64-row block, one wavefront per column with L11 in
 //     LDS (dtrsm);
 //   * C -= L U on v_mfma_f64_16x16x4f64 in 64 x 64 tiles (dgemm), k staged
@@ -734,7 +734,7 @@ namespace {
 int lu_factor(ks_ctx ctx, ks_csr A, double sigma, ks_lu *out, bool coop);
 }
 
-// The cooperative sub-panels wait on each other; should another stream's work
+// A one-launch sub-panel's workgroups wait on each other; should another stream's work
 // keep some of them from running until a wait runs out, the factorization is
 // made again with the column-step launches, which wait on nothing.
 extern "C" int ks_lu_create(ks_ctx ctx, ks_csr A, double sigma, ks_lu *out) {
@@ -793,8 +793,8 @@ int lu_factor(ks_ctx ctx, ks_csr A, double sigma, ks_lu *out, bool coop) {
   double *d_pm = (double *)((char *)scratch + off_dbl);
   unsigned long long *d_cand = (unsigned long long *)(d_pm + 2 * KS_LU_PG_MAX);
   unsigned long long *d_crow = d_cand + 2 * KS_LU_CO_MAX * KS_LU_CAND;
-  unsigned e0 = 1;     // the next cooperative sub-panel's first epoch (the words start at 0)
-  // coop: cooperative launches wanted and available (else the column-step launches)
+  unsigned e0 = 1;     // the next k_lu_panel's first epoch (the words start at 0)
+  // coop: one launch a sub-panel wanted and available (else the column-step launches)
   hipStream_t st = ctx->stream;
   const int fill_blocks = (ldn + KS_BLOCK - 1) / KS_BLOCK;
   hipLaunchKernelGGL(k_lu_fill, dim3(fill_blocks), dim3(KS_BLOCK), 0, st, A->d_rowptr, A->d_colidx,
@@ -826,7 +826,7 @@ int lu_factor(ks_ctx ctx, ks_csr A, double sigma, ks_lu *out, bool coop) {
         }
         gemm(J0, s, j0, ldn - j0, j0, KS_LU_NB);
       }
-      if (coop) {   // the sub-panel in one cooperative launch
+      if (coop) {   // the sub-panel in one launch
         const int Gc = (ldn - j0 + KS_LU_PT - 1) / KS_LU_PT;
         double *a_A = F->d_A;
         int a_ldn = ldn, a_j0 = j0;
@@ -892,7 +892,7 @@ int lu_factor(ks_ctx ctx, ks_csr A, double sigma, ks_lu *out, bool coop) {
     ks_lu_destroy(F);
     KS_HIP(herr);
   }
-  if (perr) {   // the caller makes it again without cooperative launches
+  if (perr) {   // the caller makes it again with the column-step launches
     ks_lu_destroy(F);
     return KS_ERR_TIMEOUT;
   }
