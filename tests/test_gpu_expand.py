@@ -44,7 +44,7 @@ def _expand(csr, nc, k, m, prec=0, vprec=0, refine=0, seed=0, start=None, pad=0,
             ks.check(ks.lib().ks_arnoldi_expand(ctx.h, A.h, prec, n, dV.ptr, ld, nc, a, b, buf.ptr, ldb, refine, 0.7071,
                                                 C.byref(taken)), "expand")
         out.append(ctx.status())
-    r = dV.numpy(), buf.numpy(), out[-1], taken.value
+    r = dV.numpy(), buf.numpy(), out[-1], taken.value, A.info()["nblocks"]
     A.free()
     ctx.close()
     return r
@@ -56,7 +56,7 @@ def _dense_mul(csr, X, vprec):
     return sp.csr_matrix((v, csr[1], csr[0]), shape=(len(csr[0]) - 1,) * 2) @ X
 
 
-CASES = [  # matrix, rows blocks wanted, constraints, first, last column
+CASES = [  # matrix, its row blocks (workgroups), constraints, first, last column
     (lambda: M.convection_diffusion_2d(3), 1, 0, 0, 7),
     (lambda: M.convection_diffusion_2d(16), 1, 2, 0, 33),
     (lambda: M.convection_diffusion_2d(23), 3, 0, 5, 9),
@@ -76,8 +76,8 @@ def test_expansion_in_one_launch(i, prec, vprec, refine):
     make, blocks, nc, k, m = CASES[i]
     csr = make()
     n = len(csr[0]) - 1
-    V, B, st, taken = _expand(csr, nc, k, m, prec, vprec, refine, pad=i % 3)
-    assert taken == 1 and st.error == 0 and st.breakdown_col == -1
+    V, B, st, taken, nblocks = _expand(csr, nc, k, m, prec, vprec, refine, pad=i % 3)
+    assert taken == 1 and nblocks == blocks and st.error == 0 and st.breakdown_col == -1
     assert (V[n:] == 0).all() and st.beta_last == B[nc + m, m]
     V = V[:n].astype(np.float64)
     H = B[:nc + m + 1, 1:m + 1]
