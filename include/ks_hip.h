@@ -177,13 +177,24 @@ int ks_bv_tsqr(ks_ctx ctx, int n, double *d_V, int ld, int k, int form_q, double
    ordering, its defaults), factored on the device one dependency level of rows
    at a time; A's rows must list increasing columns and hold their diagonal.
    Fails with KS_ERR_PIVOT on a zero pivot.  Applying it is one launch for each
-   factor, rows pipelined through their published values (ks_ilu0_levels gives
-   the dependency depth of each).  Replaces PCSetUp_ILU / PCApply_ILU as
+   factor: by levels in one workgroup where both factors have the layout that
+   ks_ilu0_layout describes (and there is room for it), else rows pipelined through
+   their published values; ks_ilu0_levels gives the dependency depth of each.
+   ks_bcgs_solve_ilu leaves B b in the second n doubles of its workspace.  Replaces PCSetUp_ILU / PCApply_ILU as
    KSPSolve reaches them from STApply_Sinvert
    (src/sys/classes/st/impls/sinvert/sinvert.c:16-30). */
 int ks_ilu0_create(ks_ctx ctx, ks_csr A, double sigma, ks_ilu *out);
 int ks_ilu0_destroy(ks_ilu M);
 int ks_ilu0_levels(ks_ilu M, int *nlower, int *nupper);
+/* The level-ordered layout of one factor on a pattern (host arrays; no device is
+   used): rows of a step (0: the factor has none), threads of the workgroup, entries
+   stored a row, solved values kept in LDS, and its bytes of device memory, at most
+   304 n. */
+typedef struct {
+  int step, threads, entries, ring;
+  int64_t bytes;
+} ks_ilu_layout;
+int ks_ilu0_layout(int n, const int32_t *rowptr, const int32_t *colidx, int lower, ks_ilu_layout *out);
 /* ks_bcgs_solve with the ILU(0) preconditioner B = (L U)^-1 */
 int ks_bcgs_solve_ilu(ks_ctx ctx, ks_csr A, double sigma, ks_ilu M, const double *d_b, double *d_x, double rtol,
                       double abstol, int maxits, double *d_work, int *its, double *rnorm, int *reason);

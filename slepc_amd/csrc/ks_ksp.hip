@@ -23,6 +23,7 @@
 // operation and each sum, 12.8 us so (BiCGStab 40.9 and 19.0).
 #include <algorithm>
 #include <cstring>
+#include <new>
 #include <vector>
 
 #include "ks_internal.hpp"
@@ -643,14 +644,15 @@ __global__ __launch_bounds__(KS_BLOCK) void k_ilu0_sf(int n, const int32_t *__re
 // that are deep and narrow (a grid in natural order).  k_ilu0_sf hands a value
 // from row to row through memory, about 1.3 us a level whatever the level's
 // width; here the solved values stay in a ring in LDS and a level costs an LDS
-// round trip and a barrier.  Rows are laid out in level order, NT to a step and
+// round trip and a barrier.  Rows are laid out in level order, ns to a step and
 // each level padded to whole steps (row -1), their entries in E columns of a
 // fixed width (absent: coefficient 0 on the ring's zero slot), so every load is
 // coalesced and its address known in advance: KS_ILU_PD steps are in flight in
-// registers and the barrier waits for LDS only.  A row's subtractions keep
-// k_ilu0_sf's order, so the results are its bits.
+// registers and the barrier waits for LDS only.  Threads past ns repeat the
+// step's last row and store nothing.  A row's subtractions keep k_ilu0_sf's
+// order, so the results are its bits.
 // 128 x 127 five-point grid (254 levels): one application of both factors 673
-// us by k_ilu0_sf, 114 us by levels (0.22 us a level).
+// us by k_ilu0_sf, 106 us by levels (0.21 us a level).
 #define KS_ILU_PD 8
 __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
@@ -658,17 +660,18 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 template <bool LOWER, int E, int NT>
-__global__ __launch_bounds__(NT) void k_ilu0_levels(int nsteps, int ring, const int32_t *__restrict__ rowid,
+__global__ __launch_bounds__(NT) void k_ilu0_levels(int nsteps, int ns, int ring, const int32_t *__restrict__ rowid,
                                                    const int32_t *__restrict__ dep, const double *__restrict__ coef,
                                                    const double *__restrict__ dg, double *y, const ksp_state *S) {
   if (S && S->reason) return;
   extern __shared__ double xs[];   // ring values, then the zero slot
-  const int t = threadIdx.x;
-  const int np = nsteps * NT;      // at most a few times n: below 2^31
+  const int t = threadIdx.x, ts = min(t, ns - 1);
+  const bool own = t < ns;
+  const int np = nsteps * ns;      // at most KS_ILU_PAD times n
   if (t == 0) xs[ring] = 0.0;
   int rnext[KS_ILU_PD], r[KS_ILU_PD], d[KS_ILU_PD][E];
   double c[KS_ILU_PD][E], b[KS_ILU_PD], g[KS_ILU_PD];
-  auto at = [&](int s) { return min(s, nsteps - 1) * NT + t; };
+  auto at = [&](int s) { return min(s, nsteps - 1) * ns + ts; };
   auto load = [&](int j, int s) {   // step s into slot j; its rows were loaded KS_ILU_PD steps before
     const int p = at(s);
     r[j] = rnext[j];
@@ -697,8 +700,10 @@ __global__ __launch_bounds__(NT) void k_ilu0_levels(int nsteps, int ring, const 
 #pragma unroll
       for (int e = 0; e < E; e++) x -= c[j][e] * v[e];
       if (!LOWER) x /= g[j];
-      xs[(s * NT + t) & (ring - 1)] = x;
-      if (r[j] >= 0) y[r[j]] = x;
+      if (own) {
+        xs[(s * ns + t) & (ring - 1)] = x;
+        if (r[j] >= 0) y[r[j]] = x;
+      }
       load(j, s + KS_ILU_PD);
       lds_barrier();
     }
@@ -809,7 +814,10 @@ struct ks_ilu_s {
   const int32_t *d_rowptr = nullptr, *d_colidx = nullptr;   // the operator's pattern (borrowed)
   // one factor in level order for k_ilu0_levels (nsteps 0: k_ilu0_sf takes it)
   struct lvl {
-    int nsteps = 0, nt = 0, E = 0, ring = 0;
+    int nsteps = 0, ns = 0, nt = 0, E = 0, ring = 0;
+    size_t np() const { return (size_t)nsteps * ns; }   // slots
+    size_t nidx() const { return np() * (2 * E + 1); }
+    size_t nval() const { return np() * (E + 1); }
     int32_t *d_idx = nullptr;      // rowid[np], dep[E][np], src[E][np]
     double *d_val = nullptr;       // dg[np], then coef[E][np]
   } lo, up;
@@ -823,22 +831,23 @@ namespace {
 
 template <bool LOWER, int E, int NT>
 void launch_levels(ks_ctx ctx, const ks_ilu_s::lvl &L, double *y, const ksp_state *S) {
-  const int np = L.nsteps * NT;
+  const size_t np = L.np();
   hipLaunchKernelGGL((k_ilu0_levels<LOWER, E, NT>), dim3(1), dim3(NT), sizeof(double) * (L.ring + 1), ctx->stream,
-                     L.nsteps, L.ring, (const int32_t *)L.d_idx, (const int32_t *)L.d_idx + np,
+                     L.nsteps, L.ns, L.ring, (const int32_t *)L.d_idx, (const int32_t *)L.d_idx + np,
                      (const double *)L.d_val + np, (const double *)L.d_val, y, S);
 }
 template <bool LOWER>
 void apply_levels(ks_ctx ctx, const ks_ilu_s::lvl &L, double *y, const ksp_state *S) {
-  if (L.nt == 256) {
-    if (L.E == 2) launch_levels<LOWER, 2, 256>(ctx, L, y, S);
-    else launch_levels<LOWER, 4, 256>(ctx, L, y, S);
-  } else if (L.nt == 512) {
-    if (L.E == 2) launch_levels<LOWER, 2, 512>(ctx, L, y, S);
-    else launch_levels<LOWER, 4, 512>(ctx, L, y, S);
-  } else {   // 1024 threads leave 128 VGPRs, enough for two entries a row
-    launch_levels<LOWER, 2, 1024>(ctx, L, y, S);
+#define KS_ILU_NT(X)                                           \
+  case X:                                                      \
+    if (L.E == 2) launch_levels<LOWER, 2, X>(ctx, L, y, S);    \
+    else launch_levels<LOWER, 4, X>(ctx, L, y, S);             \
+    break;
+  switch (L.nt) {
+    KS_ILU_NT(64) KS_ILU_NT(128) KS_ILU_NT(256) KS_ILU_NT(512)
+    default: launch_levels<LOWER, 2, 1024>(ctx, L, y, S);   // leaves 128 VGPRs, enough for two entries a row
   }
+#undef KS_ILU_NT
 }
 
 // y = (L U)^-1 y on the context stream: two launches, the forward and the
@@ -875,36 +884,48 @@ void group_levels(const std::vector<int> &lev, std::vector<int32_t> &rows, std::
 
 // The level-ordered layout of one factor (entries q0(i) .. q1(i)-1 of row i),
 // appended to idx: which row, which ring slots and which factor entries stand in
-// every slot.  Returns false, and the factors keep k_ilu0_sf, where a row has
-// more than KS_ILU_EMAX entries, a dependency lies further back than the ring,
-// or the levels are so wide that the steps outnumber them KS_ILU_STEPS times
-// (k_ilu0_sf has the whole chip for them).  A BiCGStab iteration (four
-// triangular solves), k_ilu0_sf / by levels: five-point grids 64 x 63 592 / 160
-// us, 128 x 127 1449 / 331, 256 x 255 7.1 / 0.84 ms, 512 x 511 48.9 / 3.0 ms;
-// seven-point grids 16^3 283 / 114 us, 64^3 (levels 1380 rows wide on average)
-// 10.7 / 2.9 ms; a tridiagonal matrix of 20,000 rows 84.8 / 20.2 ms.
+// every slot.  A step holds the widest level, up to what a workgroup takes, but
+// is halved while the padding of narrower levels makes more than KS_ILU_PAD slots a
+// row: a slot takes 44 or 76 bytes, and steps of at least 256 rows whatever the
+// levels took 22 GB for a tridiagonal matrix of 1,000,000 rows.  Returns false, and
+// the factors keep k_ilu0_sf, where a row has more than KS_ILU_EMAX entries, a
+// dependency lies further back than the ring, or the levels are so wide that the
+// steps outnumber them KS_ILU_STEPS times (k_ilu0_sf has the whole chip for them).
+// A BiCGStab iteration (four triangular solves), k_ilu0_sf / by levels: five-point
+// grids 64 x 63 592 / 118 us, 128 x 127 1449 / 236, 256 x 255 7.1 / 0.82 ms, 512 x
+// 511 48.9 / 3.0 ms; seven-point grids 16^3 283 / 97 us, 64^3 (levels 1380 rows wide
+// on average) 10.7 / 2.9 ms; a tridiagonal matrix of 20,000 rows 84.8 / 16.6 ms.
 #define KS_ILU_STEPS 4
+#define KS_ILU_PAD 4
 template <typename Q0, typename Q1>
-bool level_layout(int n, const std::vector<int32_t> &rows, const std::vector<int> &ptr, const std::vector<int32_t> &ci,
-                  Q0 q0, Q1 q1, ks_ilu_s::lvl &L, std::vector<int32_t> &idx) {
+bool level_layout(int n, const std::vector<int32_t> &rows, const std::vector<int> &ptr, const int32_t *ci, Q0 q0, Q1 q1,
+                  ks_ilu_s::lvl &L, std::vector<int32_t> &idx) {
   const int nl = (int)ptr.size() - 1;
   int emax = 0, wmax = 0;
   for (int i = 0; i < n; i++) emax = std::max(emax, (int)(q1(i) - q0(i)));
   for (int l = 0; l < nl; l++) wmax = std::max(wmax, ptr[l + 1] - ptr[l]);
   if (emax > KS_ILU_EMAX) return false;
-  const int E = emax <= 2 ? 2 : KS_ILU_EMAX, nt = wmax <= 256 ? 256 : (wmax <= 512 || E > 2 ? 512 : 1024);
-  int64_t steps = 0;
-  for (int l = 0; l < nl; l++) steps += (ptr[l + 1] - ptr[l] + nt - 1) / nt;
-  if (steps > (int64_t)KS_ILU_STEPS * nl || steps * nt * E >= (1 << 29)) return false;
-  const int np = (int)steps * nt;
+  const int E = emax <= 2 ? 2 : KS_ILU_EMAX, ntmax = E > 2 ? 512 : 1024;
+  int ns = 1;
+  while (ns < wmax && ns < ntmax) ns *= 2;
+  auto count = [&](int w) {
+    int64_t k = 0;
+    for (int l = 0; l < nl; l++) k += (ptr[l + 1] - ptr[l] + w - 1) / w;
+    return k;
+  };
+  int64_t steps = count(ns);
+  while (steps * ns > KS_ILU_PAD * (int64_t)n) steps = count(ns /= 2);   // one row a step: n slots
+  if (steps > (int64_t)KS_ILU_STEPS * nl || steps * ns * E >= (1 << 29)) return false;
+  const int np = (int)steps * ns;
   std::vector<int> pos(n);
   const size_t at = idx.size();
   idx.resize(at + (size_t)np * (2 * E + 1), -1);
   int32_t *id = idx.data() + at, *dep = id + np, *src = dep + (size_t)np * E;
-  int s = 0, ring = nt;
+  int s = 0, ring = 64;
+  while (ring < ns) ring *= 2;
   for (int l = 0; l < nl; l++) {
     for (int k = ptr[l]; k < ptr[l + 1]; k++) {
-      const int i = rows[k], p = s * nt + (k - ptr[l]), end = (p / nt + 1) * nt;
+      const int i = rows[k], p = s * ns + (k - ptr[l]), end = (p / ns + 1) * ns;
       pos[i] = p;
       id[p] = i;
       size_t e = p;
@@ -916,28 +937,69 @@ bool level_layout(int n, const std::vector<int32_t> &rows, const std::vector<int
         src[e] = q;
       }
     }
-    s += (ptr[l + 1] - ptr[l] + nt - 1) / nt;
+    s += (ptr[l + 1] - ptr[l] + ns - 1) / ns;
   }
   for (size_t k = 0; k < (size_t)np * E; k++) dep[k] = dep[k] < 0 ? ring : (dep[k] & (ring - 1));
   L.nsteps = (int)steps;
-  L.nt = nt;
+  L.ns = ns;
+  L.nt = std::max(ns, 64);
   L.E = E;
   L.ring = ring;
   return true;
 }
 
-// uploads both layouts and packs the factors' values
+// the diagonal entries of a pattern whose rows list increasing columns
+int find_diagonals(int n, const int32_t *rp, const int32_t *ci, int32_t *diag) {
+  for (int i = 0; i < n; i++) {
+    diag[i] = -1;
+    for (int32_t q = rp[i]; q < rp[i + 1]; q++) {
+      KS_CHECK(q == rp[i] || ci[q] > ci[q - 1], KS_ERR_ARG, "ILU(0) needs increasing column indices (row %d)", i);
+      if (ci[q] == i) diag[i] = q;
+    }
+    KS_CHECK(diag[i] >= 0, KS_ERR_ARG, "ILU(0) needs the diagonal entry of row %d", i);
+  }
+  return KS_OK;
+}
+
+// the rows by level and the level starts: forward (row i after the rows of its L
+// part) or backward (after its U part)
+void factor_levels(bool lower, int n, const int32_t *rp, const int32_t *ci, const int32_t *diag, std::vector<int> &lev,
+                   std::vector<int32_t> &rows, std::vector<int> &ptr) {
+  lev.assign(n, 0);
+  if (lower) {
+    for (int i = 0; i < n; i++)
+      for (int32_t q = rp[i]; q < diag[i]; q++) lev[i] = std::max(lev[i], lev[ci[q]] + 1);
+  } else {
+    for (int i = n - 1; i >= 0; i--)
+      for (int32_t q = diag[i] + 1; q < rp[i + 1]; q++) lev[i] = std::max(lev[i], lev[ci[q]] + 1);
+  }
+  group_levels(lev, rows, ptr);
+}
+
+bool factor_layout(bool lower, int n, const int32_t *rp, const int32_t *ci, const int32_t *diag,
+                   const std::vector<int32_t> &rows, const std::vector<int> &ptr, ks_ilu_s::lvl &L,
+                   std::vector<int32_t> &idx) {
+  if (lower)
+    return level_layout(n, rows, ptr, ci, [&](int i) { return rp[i]; }, [&](int i) { return diag[i]; }, L, idx);
+  return level_layout(n, rows, ptr, ci, [&](int i) { return diag[i] + 1; }, [&](int i) { return rp[i + 1]; }, L, idx);
+}
+
+// Uploads both layouts and packs the factors' values.  KS_ERR_NOMEM where there is no
+// room for them: then nothing is held or enqueued.
 int levels_pack(ks_ctx ctx, ks_ilu M, const std::vector<int32_t> &idx) {
-  size_t off = 0, val = 0;
-  KS_TRY(ks_malloc((void **)&M->d_lvl, sizeof(int32_t) * idx.size()));
+  int e = ks_malloc((void **)&M->d_lvl, sizeof(int32_t) * idx.size());
+  if (!e) e = ks_malloc((void **)&M->lo.d_val, sizeof(double) * (M->lo.nval() + M->up.nval()));
+  if (e) {
+    if (M->d_lvl) (void)ks_free(M->d_lvl);
+    M->d_lvl = nullptr;
+    return e;
+  }
   KS_HIP(hipMemcpyAsync(M->d_lvl, idx.data(), sizeof(int32_t) * idx.size(), hipMemcpyHostToDevice, ctx->stream));
-  for (ks_ilu_s::lvl *L : {&M->lo, &M->up}) val += (size_t)L->nsteps * L->nt * (L->E + 1);
-  KS_TRY(ks_malloc((void **)&M->lo.d_val, sizeof(double) * val));
-  M->up.d_val = M->lo.d_val + (size_t)M->lo.nsteps * M->lo.nt * (M->lo.E + 1);
+  M->lo.d_idx = M->d_lvl;
+  M->up.d_idx = M->d_lvl + M->lo.nidx();
+  M->up.d_val = M->lo.d_val + M->lo.nval();
   for (ks_ilu_s::lvl *L : {&M->lo, &M->up}) {
-    const int np = L->nsteps * L->nt;
-    L->d_idx = M->d_lvl + off;
-    off += (size_t)np * (2 * L->E + 1);
+    const int np = (int)L->np();
     hipLaunchKernelGGL(k_ilu0_pack, dim3(ksp_blocks(np)), dim3(KS_BLOCK), 0, ctx->stream, np, L->E,
                        (const int32_t *)L->d_idx + (size_t)np * (L->E + 1), (const int32_t *)L->d_idx,
                        (const int32_t *)M->d_diag, (const double *)M->d_lu, L->d_val + np, L->d_val);
@@ -954,32 +1016,19 @@ int ks_ilu0_create(ks_ctx ctx, ks_csr A, double sigma, ks_ilu *out) {
   *out = nullptr;
   const int n = A->nrows;
   const int64_t nnz = A->nnz;
-  std::vector<int32_t> rp(n + 1), ci(nnz), diag(n, -1);
+  std::vector<int32_t> rp(n + 1), ci(nnz), diag(n);
   KS_HIP(hipMemcpyAsync(rp.data(), A->d_rowptr, sizeof(int32_t) * (n + 1), hipMemcpyDeviceToHost, ctx->stream));
   KS_HIP(hipMemcpyAsync(ci.data(), A->d_colidx, sizeof(int32_t) * nnz, hipMemcpyDeviceToHost, ctx->stream));
   KS_HIP(hipStreamSynchronize(ctx->stream));
-  // the pattern's rows must list increasing columns and hold their diagonal
-  for (int i = 0; i < n; i++) {
-    for (int32_t q = rp[i]; q < rp[i + 1]; q++) {
-      KS_CHECK(q == rp[i] || ci[q] > ci[q - 1], KS_ERR_ARG, "ILU(0) needs increasing column indices (row %d)", i);
-      if (ci[q] == i) diag[i] = q;
-    }
-    KS_CHECK(diag[i] >= 0, KS_ERR_ARG, "ILU(0) needs the diagonal entry of row %d", i);
-  }
-  // levels: forward (row i after the rows of its L part), backward (after its U part)
-  std::vector<int> lev(n, 0);
-  for (int i = 0; i < n; i++)
-    for (int32_t q = rp[i]; q < diag[i]; q++) lev[i] = lev[ci[q]] + 1 > lev[i] ? lev[ci[q]] + 1 : lev[i];
+  KS_TRY(find_diagonals(n, rp.data(), ci.data(), diag.data()));
+  std::vector<int> lev;
+  std::vector<int32_t> lrows, urows;
   ks_ilu M = new ks_ilu_s();
   M->n = n;
   M->d_rowptr = A->d_rowptr;
   M->d_colidx = A->d_colidx;
-  std::vector<int32_t> lrows, urows;
-  group_levels(lev, lrows, M->lptr);
-  std::fill(lev.begin(), lev.end(), 0);
-  for (int i = n - 1; i >= 0; i--)
-    for (int32_t q = diag[i] + 1; q < rp[i + 1]; q++) lev[i] = lev[ci[q]] + 1 > lev[i] ? lev[ci[q]] + 1 : lev[i];
-  group_levels(lev, urows, M->uptr);
+  factor_levels(true, n, rp.data(), ci.data(), diag.data(), lev, lrows, M->lptr);
+  factor_levels(false, n, rp.data(), ci.data(), diag.data(), lev, urows, M->uptr);
   int e = KS_OK;
   // the rows by level and the level starts
   lrows.insert(lrows.end(), M->lptr.begin(), M->lptr.end());
@@ -1015,18 +1064,25 @@ int ks_ilu0_create(ks_ctx ctx, ks_csr A, double sigma, ks_ilu *out) {
     }
   }
   KS_HIP(hipGetLastError());
-  // the level-ordered layouts, made while the device factors
+  // The level-ordered layouts, made while the device factors; without room for them,
+  // here or on the device, the rows wait for each other (k_ilu0_sf)
   std::vector<int32_t> idx;
-  const bool by_levels =
-      level_layout(n, lrows, M->lptr, ci, [&](int i) { return rp[i]; }, [&](int i) { return diag[i]; }, M->lo, idx) &&
-      level_layout(n, urows, M->uptr, ci, [&](int i) { return diag[i] + 1; }, [&](int i) { return rp[i + 1]; }, M->up,
-                   idx);
-  if (!by_levels) M->lo.nsteps = M->up.nsteps = 0;
-  else if ((e = levels_pack(ctx, M, idx))) {
-    (void)hipStreamSynchronize(st);
-    ks_ilu0_destroy(M);
-    return e;
+  bool by_levels = false;
+  try {
+    by_levels = factor_layout(true, n, rp.data(), ci.data(), diag.data(), lrows, M->lptr, M->lo, idx) &&
+                factor_layout(false, n, rp.data(), ci.data(), diag.data(), urows, M->uptr, M->up, idx);
+  } catch (const std::bad_alloc &) {
   }
+  if (by_levels) {
+    e = levels_pack(ctx, M, idx);
+    if (e && e != KS_ERR_NOMEM) {
+      (void)hipStreamSynchronize(st);
+      ks_ilu0_destroy(M);
+      return e;
+    }
+    by_levels = !e;
+  }
+  if (!by_levels) M->lo.nsteps = M->up.nsteps = 0;
   // the last pivot, and a zero pivot met on the way
   int flag = 0;
   double ulast = 0.0;
@@ -1052,6 +1108,27 @@ int ks_ilu0_destroy(ks_ilu M) {
   if (M->d_lvl) (void)ks_free(M->d_lvl);
   if (M->lo.d_val) (void)ks_free(M->lo.d_val);
   delete M;
+  return KS_OK;
+}
+
+int ks_ilu0_layout(int n, const int32_t *rowptr, const int32_t *colidx, int lower, ks_ilu_layout *out) {
+  KS_CHECK(n > 0 && rowptr && colidx && out, KS_ERR_ARG, "bad ILU layout arguments");
+  *out = ks_ilu_layout{};
+  try {
+    std::vector<int32_t> diag(n), rows, idx;
+    std::vector<int> lev, ptr;
+    ks_ilu_s::lvl L;
+    KS_TRY(find_diagonals(n, rowptr, colidx, diag.data()));
+    factor_levels(lower != 0, n, rowptr, colidx, diag.data(), lev, rows, ptr);
+    if (!factor_layout(lower != 0, n, rowptr, colidx, diag.data(), rows, ptr, L, idx)) return KS_OK;
+    out->step = L.ns;
+    out->threads = L.nt;
+    out->entries = L.E;
+    out->ring = L.ring;
+    out->bytes = (int64_t)(sizeof(int32_t) * L.nidx() + sizeof(double) * L.nval());
+  } catch (const std::bad_alloc &) {
+    return KS_ERR_NOMEM;
+  }
   return KS_OK;
 }
 
