@@ -558,11 +558,16 @@ __global__ __launch_bounds__(64) void k_ilu0_factor_level(const int32_t *__restr
   if (t < cnt) ilu0_factor_row(rows[t], rowptr, colidx, diag, lu, zero_pivot);
 }
 
-// every level in one workgroup, a barrier (which orders its global stores)
-// between them: for levels of at most KS_ILU_WG rows a launch a level costs
-// more than the level (128 x 127 grid, 254 levels: the whole set-up takes 3.1 ms
-// with a launch a level, 1.9 ms with one launch)
-#define KS_ILU_WG 1024
+// Every level in one workgroup, a barrier (which orders its global stores) between
+// them: for narrow levels of short rows a launch a level costs more than the level.
+// Wider levels, or rows whose chains of merges are long, are better spread over the
+// chip.  The whole set-up, a launch a level / one launch: 128 x 127 grid 1.83 / 1.56
+// ms, 256 x 255 (levels of up to 255 rows) 4.35 / 4.14, 512 x 511 (511) 10.9 / 11.8,
+// tridiagonal 2,000 rows 5.3 / 2.7; nine-point 100 x 100 4.45 / 4.07; seven-point 16^3
+// (192) 0.62 / 0.57, 32^3 (768) 1.58 / 1.95; 27-point 40^3 33 / 44; random graphs of 20
+// entries a row 9.6 / 10.1.
+#define KS_ILU_WG 256        // rows of a level, at most
+#define KS_ILU_WG_ROW 9      // entries of a row, at most
 __global__ __launch_bounds__(KS_ILU_WG) void k_ilu0_factor(const int32_t *__restrict__ rows,
                                                           const int32_t *__restrict__ lptr, int nlev,
                                                           const int32_t *__restrict__ rowptr,
@@ -1049,9 +1054,10 @@ int ks_ilu0_create(ks_ctx ctx, ks_csr A, double sigma, ks_ilu *out) {
   hipLaunchKernelGGL(k_ilu0_init, dim3(ksp_blocks(n)), dim3(KS_BLOCK), 0, st, A->d_rowptr, A->d_colidx,
                      (const double *)A->d_val, n, sigma, M->d_lu);
   const int nlev = (int)M->lptr.size() - 1;
-  int wmax = 0;
+  int wmax = 0, emax = 0;
   for (int l = 0; l < nlev; l++) wmax = std::max(wmax, M->lptr[l + 1] - M->lptr[l]);
-  if (wmax <= KS_ILU_WG) {
+  for (int i = 0; i < n; i++) emax = std::max(emax, rp[i + 1] - rp[i]);
+  if (wmax <= KS_ILU_WG && emax <= KS_ILU_WG_ROW) {
     hipLaunchKernelGGL(k_ilu0_factor, dim3(1), dim3(KS_ILU_WG), 0, st, (const int32_t *)M->d_lrows,
                        (const int32_t *)M->d_lrows + n, nlev, A->d_rowptr, A->d_colidx, (const int32_t *)M->d_diag,
                        M->d_lu, M->d_flag);
