@@ -295,6 +295,9 @@ int ks_bv_orthonormalize_resume(ks_ctx ctx, ks_prec prec, int n, void *V, int ld
    column k and those before it are as they were. */
 int ks_arnoldi_expand(ks_ctx ctx, ks_csr A, ks_prec prec, int n, void *V, int ld, int nc, int k, int m,
                       double *d_buf, int ldbuf, ks_refine refine, double eta, int *taken);
+/* The polls (of about half a microsecond) after which a wait of the context's
+   ks_arnoldi_expand gives up, 0: its own bound of 2^18; a test of the recovery sets 1. */
+int ks_ctx_expand_polls(ks_ctx ctx, int polls);
 /* Reset the status for a new expansion (active=1, breakdown_col=-1). */
 int ks_status_reset(ks_ctx ctx);
 /* Copy the status to the host (synchronizes the stream). */

@@ -17,9 +17,10 @@
 // between two areas, and a workgroup writes an area again two exchanges later, when it
 // has seen the sums of the exchange between, which every workgroup gave after reading
 // the first; the vector's words are rewritten a step later, after that step's dots.
-// Every wait is bounded (KS_EXP_SPIN polls, or sooner once *err shows another ran out):
-// then the status carries KS_ERR_TIMEOUT, every workgroup leaves the kernel, and the
-// caller expands with the launches (the start column and those before it are not
+// Every wait is bounded (KS_EXP_SPIN polls unless ks_ctx_expand_polls says otherwise, or
+// sooner once *err shows another ran out): then the status carries KS_ERR_TIMEOUT, no
+// total goes out that a value is missing from, every workgroup leaves the kernel, and
+// the caller expands with the launches (the start column and those before it are not
 // touched).  The workgroups wait on each other, so they must be able to run at the
 // same time: up to KS_EXP_MAXG2 of them two fit a CU, up to KS_EXP_MAXG three, so that
 // one launch of each of the four hardware queues HIP uses fits the chip.
@@ -41,7 +42,7 @@ namespace {
 static_assert(KS_SPMV_ROWS == KS_BLOCK, "a thread a row");
 
 struct exp_args {
-  int n, ld, nc, j0, m, G;
+  int n, ld, nc, j0, m, G, polls;
   const int32_t *blk, *rowptr, *colidx;
   const void *val;
   void *V;
@@ -56,11 +57,11 @@ struct exp_args {
 
 // *err == launch: another wait of this launch has run out
 __device__ __forceinline__ double exp_wait(const unsigned long long *w, unsigned epoch, unsigned *err, unsigned launch,
-                                           int &dead) {
+                                           int polls, int &dead) {
   for (int spins = 0; !dead;) {
     const unsigned long long lo = ks_pub_load(w), hi = ks_pub_load(w + 1);
     if ((unsigned)(lo >> 32) == epoch && (unsigned)(hi >> 32) == epoch) return ks_pub_f64(lo, hi);
-    if (++spins > KS_EXP_SPIN ||
+    if (++spins > polls ||
         ((spins & 255) == 0 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == launch)) {
       __hip_atomic_store(err, launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       dead = 1;
@@ -174,7 +175,7 @@ __global__ __launch_bounds__(KS_BLOCK, WGS) void k_expand(exp_args a) {
             ok = ok && (unsigned)(lo >> 32) == ep && (unsigned)(hi >> 32) == ep;
           }
           if (ok) break;
-          if (++spins > KS_EXP_SPIN || ((spins & 255) == 0 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == launch)) {
+          if (++spins > a.polls || ((spins & 255) == 0 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == launch)) {
             __hip_atomic_store(err, launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             dead = 1;
             break;
@@ -233,7 +234,7 @@ __global__ __launch_bounds__(KS_BLOCK, WGS) void k_expand(exp_args a) {
         for (int c = wave * cpl; c <= kk; c += KS_WAVES * cpl) {
           const int cc = c + cs;
           double s = 0.0;
-          if (cc <= kk && g < G) s = exp_wait(P + 2 * ((size_t)cc * G + g), ep, err, launch, dead);
+          if (cc <= kk && g < G) s = exp_wait(P + 2 * ((size_t)cc * G + g), ep, err, launch, a.polls, dead);
           s = group_sum(s, GP);
           if (g == 0 && cc <= kk) tot[cc] = s;
         }
@@ -244,11 +245,11 @@ __global__ __launch_bounds__(KS_BLOCK, WGS) void k_expand(exp_args a) {
           double s = 0.0;
 #pragma unroll
           for (int q = 0; q < KS_EXP_MAXG / 64; q++)
-            if (lane + 64 * q < G) s += exp_wait(P + 2 * ((size_t)c * G + lane + 64 * q), ep, err, launch, dead);
+            if (lane + 64 * q < G) s += exp_wait(P + 2 * ((size_t)c * G + lane + 64 * q), ep, err, launch, a.polls, dead);
           s = ks_wave_sum(s);
-          if (lane == 0 && !dead) ks_pub_store_f64(Q + 2 * c, ep, s);
+          if (!__any(dead) && lane == 0) ks_pub_store_f64(Q + 2 * c, ep, s);
         }
-        if (tid <= kk) tot[tid] = exp_wait(Q + 2 * tid, ep, err, launch, dead);
+        if (tid <= kk) tot[tid] = exp_wait(Q + 2 * tid, ep, err, launch, a.polls, dead);
       }
       if (__syncthreads_or(dead)) break;
       // ---- the decisions of BVOrthogonalizeGS (bvorthog.c:91-217), alike in every workgroup
@@ -384,6 +385,12 @@ int exp_areas(ks_ctx ctx, unsigned long long **w) {
 
 }  // namespace
 
+extern "C" int ks_ctx_expand_polls(ks_ctx ctx, int polls) {
+  KS_CHECK(ctx && polls >= 0, KS_ERR_ARG, "bad number of polls");
+  ctx->exp_polls = polls;
+  return KS_OK;
+}
+
 extern "C" int ks_arnoldi_expand(ks_ctx ctx, ks_csr A, ks_prec prec, int n, void *V, int ld, int nc, int k, int m,
                                  double *d_buf, int ldbuf, ks_refine refine, double eta, int *taken) {
   KS_CHECK(ctx && A && V && d_buf && taken, KS_ERR_ARG, "null expansion argument");
@@ -402,6 +409,7 @@ extern "C" int ks_arnoldi_expand(ks_ctx ctx, ks_csr A, ks_prec prec, int n, void
   a.j0 = k;
   a.m = m;
   a.G = A->nblocks;
+  a.polls = ctx->exp_polls ? ctx->exp_polls : KS_EXP_SPIN;
   a.blk = A->d_blk;
   a.rowptr = A->d_rowptr;
   a.colidx = A->d_colidx;

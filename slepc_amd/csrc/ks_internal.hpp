@@ -103,6 +103,7 @@ struct ks_ctx_s {
   ks_status *h_status = nullptr;   // pinned mirror of d_status, filled by ks_status_post
   unsigned long long *d_exp = nullptr;      // the exchange areas of ks_arnoldi_expand, and ...
   unsigned exp_epoch = 0;                   // ... the next launch's first epoch
+  int exp_polls = 0;                        // ks_ctx_expand_polls
   // a call's workspace, kept for the next call on the context (ks_ws_take)
   void *d_ws = nullptr;
   size_t ws_bytes = 0;

@@ -132,3 +132,82 @@ def test_left_to_the_launches():
     rp = np.concatenate([[0, n], n + np.arange(1, n)]).astype(np.int32)
     ci = np.concatenate([np.arange(n), np.arange(1, n)]).astype(np.int32)
     assert _expand((rp, ci, np.ones(2 * n - 1)), 0, 0, 4)[3] == 0
+
+
+@pytest.mark.parametrize("side,blocks,nc", [(23, 3, 1), (65, 17, 0), (182, 130, 2)])
+def test_wait_that_runs_out(side, blocks, nc):
+    """Waits that give up at their second poll: the status says so, every workgroup leaves, column
+    k and those before it stay, and the context's next expansion is that of a new context."""
+    from slepc_amd import ks
+    csr = M.convection_diffusion_2d(side)
+    n, k, m = side * side, 3, 24
+    L, ldb = ks.lib(), nc + m + 2
+    V0 = np.zeros((n, nc + m + 1), order="F")
+    V0[:, :nc + 1] = np.linalg.qr(np.random.default_rng(side).standard_normal((n, nc + 1)))[0]
+    taken, out = C.c_int(), []
+    for disturb in (False, True):
+        ctx = ks.Context()
+        A = ks.CSR(ctx, csr)
+        assert A.info()["nblocks"] == blocks
+        dV, buf = ks.DeviceArray.from_numpy(ctx, V0), ks.DeviceArray.from_numpy(ctx, np.zeros((ldb, m + 1), order="F"))
+
+        def expand(a, b):
+            ctx.status_reset()
+            ks.check(L.ks_arnoldi_expand(ctx.h, A.h, 0, n, dV.ptr, n, nc, a, b, buf.ptr, ldb, 0, 0.7071, C.byref(taken)),
+                     "expand")
+            assert taken.value == 1
+            return ctx.status()
+        assert expand(0, k).error == 0
+        if disturb:
+            V, B = dV.numpy(), buf.numpy()
+            ks.check(L.ks_ctx_expand_polls(ctx.h, 1), "polls")
+            st = expand(k, m)
+            assert st.error == -8 and st.active == 0
+            assert np.array_equal(dV.numpy()[:, :nc + k + 1], V[:, :nc + k + 1])
+            assert np.array_equal(buf.numpy()[:, :k + 1], B[:, :k + 1])
+            ks.check(L.ks_ctx_expand_polls(ctx.h, 0), "polls")
+        st = expand(k, m)
+        assert st.error == 0 and st.breakdown_col == -1
+        out.append((dV.numpy(), buf.numpy(), st.total_passes))
+        A.free()
+        ctx.close()
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1]) and out[0][2] == out[1][2]
+
+
+@pytest.mark.parametrize("side,nc", [(23, 2), (65, 0)])
+def test_expansion_again_by_the_launches(side, nc):
+    """BVMatArnoldi whose one launch gives up returns what the launches give, bit for bit, in that
+    expansion and in the basis' next one."""
+    from slepc_amd import eps as E
+    from slepc_amd import ks
+    n, k, m = side * side, 9, 20
+    rng = np.random.default_rng(side)
+    start, cons = rng.standard_normal(n), rng.standard_normal((n, max(nc, 1)))
+    A = E.Mat(M.convection_diffusion_2d(side))
+    out = {}
+    for form in ("one launch", "launches", "again"):
+        bv = E.BV(n, m + 1)
+        if nc:
+            assert bv.insert_constraints(cons) == nc      # makes the basis' storage again
+        E._chk(E.lib().BVHIPKSSetOneLaunch(bv.h, C.c_int(form != "launches")), "BVHIPKSSetOneLaunch")
+        bv.set_columns((start / np.linalg.norm(start))[:, None])
+        E._chk(E.lib().BVOrthonormalizeColumn(bv.h, C.c_int(0), C.c_int(0), None, None), "BVOrthonormalizeColumn")
+        got = []
+        try:
+            ks.check(ks.lib().ks_ctx_expand_polls(E.context_handle(), int(form == "again")), "polls")
+            for a, b in ((0, k), (k, m)):
+                H, h = E.BV._dense(m + 1, m)
+                mm, beta, brk = C.c_int(b), C.c_double(), C.c_int()
+                E._chk(E.lib().BVMatArnoldi(bv.h, A.h, h, C.c_int(a), C.byref(mm), C.byref(beta), C.byref(brk)),
+                       "BVMatArnoldi")
+                assert mm.value == b and not brk.value
+                got += [H[:, a:b].copy(), beta.value]
+                E.lib().MatDestroy(C.byref(h))
+        finally:
+            ks.check(ks.lib().ks_ctx_expand_polls(E.context_handle(), 0), "polls")
+        out[form] = got + [bv.get_columns()]
+        bv.destroy()
+    A.destroy()
+    assert not np.array_equal(out["one launch"][-1], out["launches"][-1])     # the sums of the two are ordered differently
+    for a, b in zip(out["again"], out["launches"]):
+        assert np.array_equal(a, b)
