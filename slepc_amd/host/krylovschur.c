@@ -59,11 +59,6 @@ static PetscErrorCode EPSAllocateSolution(EPS eps, PetscInt extra)
   if (!strcmp(BVTypeName(V), BVHIPKS)) {
     PetscCall(BVHIPKSSetStepGraphs(V, ctx->step_graphs));
     PetscCall(BVHIPKSSetGrouped(V, ctx->grouped));
-    /* a harmonic restart's vector (u - V g) / gamma carries the expansion's rounding times
-       1 / gamma, some 1e6: results to a tolerance near that stay those of the launches' order
-       of sums (laplacian of 200 rows, target 1, tol 1e-10: eigenvalues good to 2e-11 in that
-       order, to 9e-11 in the one launch's, the other way round for other start vectors) */
-    PetscCall(BVHIPKSSetOneLaunch(V, (PetscBool)(eps->extraction != EPS_HARMONIC || eps->twosided)));
   }
   /* W: a basis like V for the two-sided variant (epssetup.c:726-731) */
   if (eps->W && (!eps->twosided || eps->W->m != requested || eps->W->n != eps->n || strcmp(eps->W->vtype, V->vtype)))
@@ -749,6 +744,13 @@ static PetscErrorCode EPSSolveBegin_KrylovSchur(EPS eps)
   ctx->its32 = ctx->nconv32 = 0;
   ctx->nmatmult32 = ctx->passes32 = 0;
   ctx->t32 = 0.0;
+  /* Harmonic solves keep the launches' order of sums: a harmonic restart's vector
+     (u - V g) / gamma carries the expansion's rounding times 1 / gamma, up to 1e6 where the
+     target is an eigenvalue.  Over 40 start vectors each, laplacian of 200 rows, tol 1e-10,
+     target 1 and 3 (eigenvalues): errors alike on average (4e-11), the worst 2e-10 and 1e-10
+     by the launches, 6e-10 and 2e-9 by the one launch; six other problems show no difference.
+     Set here and not with the basis, whose storage deflation vectors make again. */
+  if (!strcmp(BVTypeName(eps->V), BVHIPKS)) PetscCall(BVHIPKSSetOneLaunch(eps->V, (PetscBool)!ctx->harmonic));
   if (eps->twosided) return TSStart(eps);
   if (ctx->mixed_tol > 0.0 && ctx->mixed_tol > eps->tol && BVPrecision(eps->V) == SLEPC_AMD_F64) return MixedBegin(eps);
   return KSStart(eps);

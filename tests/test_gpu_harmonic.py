@@ -107,6 +107,23 @@ def test_interior_at_device_size_vs_oracle(E, oracle):
     assert (r["err"][:4] <= 1e-10).all()
 
 
+def test_deflated_harmonic_solve_keeps_the_launches(E):
+    # the deflation vector makes the basis' storage again; per-kernel events rule the one launch out
+    from slepc_amd import ks
+    n = 200
+    csr = M.laplacian_1d(n)
+    d = np.random.default_rng(4).standard_normal((n, 1))
+    out = []
+    for events in (0, 1):
+        ks.check(ks.lib().ks_prof_enable(E.context_handle(), events), "ks_prof_enable")
+        try:
+            out.append(E.solve(csr, nev=4, ncv=24, tol=1e-9, target=1.5, which=E.EPS.TARGET_MAGNITUDE,
+                               extraction=E.EPS.HARMONIC, deflation=d, v0=M.uniform_vector(8, n)))
+        finally:
+            ks.check(ks.lib().ks_prof_enable(E.context_handle(), 0), "ks_prof_enable")
+    assert out[0]["its"] == out[1]["its"] and np.array_equal(out[0]["eigr"], out[1]["eigr"])
+
+
 def test_unsupported_extraction_is_refused(E):
     A = E.Mat(M.laplacian_1d(50))
     eps = E.EPS()
