@@ -290,7 +290,7 @@ int ks_bv_orthonormalize_resume(ks_ctx ctx, ks_prec prec, int n, void *V, int ld
    reset; it reports breakdown and the last norm as after the launches.  *taken = 0
    (and nothing enqueued) where the launches are the way: more than 192 row
    blocks, a row longer than a row block, more than 128 columns, m >= n, events
-   or a capture on the context.  A status error of KS_ERR_TIMEOUT (its
+   or a capture on the context, no room for its 0.9 MB.  A status error of KS_ERR_TIMEOUT (its
    workgroups could not run at the same time): expand again by the launches,
    column k and those before it are as they were. */
 int ks_arnoldi_expand(ks_ctx ctx, ks_csr A, ks_prec prec, int n, void *V, int ld, int nc, int k, int m,

@@ -368,11 +368,16 @@ __global__ __launch_bounds__(KS_BLOCK, WGS) void k_expand(exp_args a) {
   }
 }
 
-// the exchange areas of a context, made by its first expansion: the epochs of its words start at 0
+// the exchange areas of a context, made by its first expansion (none: there is no room for them);
+// the epochs of its words start at 0
 int exp_areas(ks_ctx ctx, unsigned long long **w) {
   const size_t words = 2 * (2 * (size_t)(KS_EXP_MAXK + 1) * (KS_EXP_MAXG + 1) + (size_t)KS_EXP_MAXG * KS_SPMV_ROWS) + 8;
   if (!ctx->d_exp) {
-    KS_HIP(hipMalloc((void **)&ctx->d_exp, words * sizeof(unsigned long long)));
+    if (hipMalloc((void **)&ctx->d_exp, words * sizeof(unsigned long long)) != hipSuccess) {
+      (void)hipGetLastError();
+      *w = ctx->d_exp = nullptr;
+      return KS_OK;
+    }
     ctx->exp_epoch = 0;
   }
   if (ctx->exp_epoch == 0 || ctx->exp_epoch > 0xf0000000u) {
@@ -403,6 +408,7 @@ extern "C" int ks_arnoldi_expand(ks_ctx ctx, ks_csr A, ks_prec prec, int n, void
   exp_args a = {};
   unsigned long long *w;
   KS_TRY(exp_areas(ctx, &w));
+  if (!w) return KS_OK;
   a.n = n;
   a.ld = ld;
   a.nc = nc;
