@@ -290,13 +290,16 @@ int ks_bv_orthonormalize_resume(ks_ctx ctx, ks_prec prec, int n, void *V, int ld
    reset; it reports breakdown and the last norm as after the launches.  *taken = 0
    (and nothing enqueued) where the launches are the way: more than 192 row
    blocks, a row longer than a row block, more than 128 columns, m >= n, events
-   or a capture on the context, no room for its 0.9 MB.  A status error of KS_ERR_TIMEOUT (its
+   or a capture on the context, no room for its 1.6 MB, or a wait
+   that ran out not long ago.  A status error of KS_ERR_TIMEOUT (its
    workgroups could not run at the same time): expand again by the launches,
    column k and those before it are as they were. */
 int ks_arnoldi_expand(ks_ctx ctx, ks_csr A, ks_prec prec, int n, void *V, int ld, int nc, int k, int m,
                       double *d_buf, int ldbuf, ks_refine refine, double eta, int *taken);
 /* The polls (of about half a microsecond) after which a wait of the context's
-   ks_arnoldi_expand gives up, 0: its own bound of 2^18; a test of the recovery sets 1. */
+   ks_arnoldi_expand gives up, 0: its own bound of 2^18; a test of the recovery sets 1.
+   After a wait that ran out the context's next 16 expansions are left to the launches,
+   twice as many after each further one, up to 4,096; setting the polls forgets it. */
 int ks_ctx_expand_polls(ks_ctx ctx, int polls);
 /* Reset the status for a new expansion (active=1, breakdown_col=-1). */
 int ks_status_reset(ks_ctx ctx);

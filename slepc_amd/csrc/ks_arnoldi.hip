@@ -21,7 +21,9 @@
 // sooner once *err shows another ran out): then the status carries KS_ERR_TIMEOUT, no
 // total goes out that a value is missing from, every workgroup leaves the kernel, and
 // the caller expands with the launches (the start column and those before it are not
-// touched).  The workgroups wait on each other, so they must be able to run at the
+// touched).  Beside work that keeps the chip full each such launch costs 0.1 s and more,
+// so the context then leaves a growing number of expansions to the launches at once.
+// The workgroups wait on each other, so they must be able to run at the
 // same time: up to KS_EXP_MAXG2 of them two fit a CU, up to KS_EXP_MAXG three, so that
 // one launch of each of the four hardware queues HIP uses fits the chip.
 #include "ks_internal.hpp"
@@ -393,6 +395,7 @@ int exp_areas(ks_ctx ctx, unsigned long long **w) {
 extern "C" int ks_ctx_expand_polls(ks_ctx ctx, int polls) {
   KS_CHECK(ctx && polls >= 0, KS_ERR_ARG, "bad number of polls");
   ctx->exp_polls = polls;
+  ctx->exp_hold = ctx->exp_back = 0;
   return KS_OK;
 }
 
@@ -405,6 +408,10 @@ extern "C" int ks_arnoldi_expand(ks_ctx ctx, ks_csr A, ks_prec prec, int n, void
   *taken = 0;
   if (ctx->prof || ctx->capturing) return KS_OK;   // per-kernel events, or a replay that would repeat the epochs
   if (A->variant != 0 || A->nblocks > KS_EXP_MAXG || nc + m > KS_EXP_MAXK || m > n - 1) return KS_OK;
+  if (ctx->exp_hold > 0) {   // a launch's workgroups could not all run (ks_status_get)
+    ctx->exp_hold--;
+    return KS_OK;
+  }
   exp_args a = {};
   unsigned long long *w;
   KS_TRY(exp_areas(ctx, &w));
@@ -445,6 +452,7 @@ extern "C" int ks_arnoldi_expand(ks_ctx ctx, ks_csr A, ks_prec prec, int n, void
   else KS_EXP_LAUNCH(float, float);
 #undef KS_EXP_LAUNCH
   KS_HIP(hipGetLastError());
+  ctx->exp_live = true;
   *taken = 1;
   return KS_OK;
 }

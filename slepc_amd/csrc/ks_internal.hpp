@@ -104,6 +104,8 @@ struct ks_ctx_s {
   unsigned long long *d_exp = nullptr;      // the exchange areas of ks_arnoldi_expand, and ...
   unsigned exp_epoch = 0;                   // ... the next launch's first epoch
   int exp_polls = 0;                        // ks_ctx_expand_polls
+  bool exp_live = false;                    // the status of an expansion's launch has not been read
+  int exp_hold = 0, exp_back = 0;           // expansions left to the launches, and how many after the last time-out
   // a call's workspace, kept for the next call on the context (ks_ws_take)
   void *d_ws = nullptr;
   size_t ws_bytes = 0;

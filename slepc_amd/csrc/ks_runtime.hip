@@ -371,11 +371,21 @@ int ks_status_reset(ks_ctx c) {
   return KS_OK;
 }
 
+// the status of an expansion in one launch: after a wait that ran out the next ones on
+// the context do not try
+static void note_expansion(ks_ctx c, const ks_status *st) {
+  if (!c->exp_live) return;
+  c->exp_live = false;
+  c->exp_back = st->error != KS_ERR_TIMEOUT ? 0 : c->exp_back == 0 ? 16 : c->exp_back >= 2048 ? 4096 : 2 * c->exp_back;
+  c->exp_hold = c->exp_back;
+}
+
 int ks_status_get(ks_ctx c, ks_status *out) {
   KS_CHECK(c && out, KS_ERR_ARG, "null argument");
   KS_HIP(hipMemcpyAsync(c->h_scalar, c->d_status, sizeof(ks_status), hipMemcpyDeviceToHost, c->stream));
   KS_HIP(hipStreamSynchronize(c->stream));
   memcpy(out, c->h_scalar, sizeof(ks_status));
+  note_expansion(c, out);
   return KS_OK;
 }
 
@@ -391,6 +401,7 @@ int ks_status_read(ks_ctx c, ks_status *out) {
   KS_CHECK(c && out, KS_ERR_ARG, "null argument");
   KS_HIP(hipStreamSynchronize(c->stream));
   memcpy(out, c->h_status, sizeof(ks_status));
+  note_expansion(c, out);
   return KS_OK;
 }
 

@@ -211,3 +211,29 @@ def test_expansion_again_by_the_launches(side, nc):
     assert not np.array_equal(out["one launch"][-1], out["launches"][-1])     # the sums of the two are ordered differently
     for a, b in zip(out["again"], out["launches"]):
         assert np.array_equal(a, b)
+
+
+def test_context_rests_after_a_wait_that_ran_out():
+    # 16 expansions by the launches, 32 after the next time-out
+    from slepc_amd import ks
+    csr, n = M.convection_diffusion_2d(65), 65 * 65
+    ctx, L, taken = ks.Context(), ks.lib(), C.c_int()
+    A = ks.CSR(ctx, csr)
+    V = ks.DeviceArray.from_numpy(ctx, np.asfortranarray(np.random.default_rng(0).standard_normal((n, 31))))
+    buf = ks.DeviceArray.from_numpy(ctx, np.zeros((32, 31), order="F"))
+
+    def expand():
+        ctx.status_reset()
+        ks.check(L.ks_arnoldi_expand(ctx.h, A.h, 0, n, V.ptr, n, 0, 0, 30, buf.ptr, 32, 0, 0.7071, C.byref(taken)), "expand")
+        return ctx.status().error if taken.value else None
+
+    def polls(k):
+        ks.check(L.ks_ctx_expand_polls(ctx.h, k), "polls")
+    polls(1)
+    assert [expand() for _ in range(18 + 33)] == [-8] + 16 * [None] + [-8] + 32 * [None] + [-8]
+    polls(0)
+    assert expand() == 0                                   # setting the polls forgets it
+    polls(1)
+    assert [expand() for _ in range(18)] == [-8] + 16 * [None] + [-8]
+    A.free()
+    ctx.close()
