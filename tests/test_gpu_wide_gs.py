@@ -1,6 +1,7 @@
 """Gram-Schmidt against more than 128 columns (the sweep of eight wavefronts): every column
 split and both sides of its lines, ragged rows, FP64 and FP32 with aligned and odd strides,
-the full and the lean sequence, against two CGS passes in numpy."""
+the full and the lean sequence, against two CGS passes in numpy; and columns of 4 GiB and more,
+whose rows need 64-bit offsets (k_gs_lds), against two passes in torch."""
 import ctypes as C
 
 import numpy as np
@@ -52,3 +53,53 @@ def test_wide_orthonormalization(k, prec, pad):
     assert abs(na - np.linalg.norm(x)) <= 30 * eps * np.linalg.norm(x)
     assert np.linalg.norm(a[:n, k] - x / np.linalg.norm(x)) <= 30 * eps
     ctx.close()
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+def test_columns_of_four_gib(prec):
+    import torch
+
+    from slepc_amd import ks
+    n, k = (2 ** 29 if prec == 0 else 2 ** 30) + 77, 3
+    ld = n + 1
+    V = torch.zeros((k + 1, ld), dtype=torch.float64 if prec == 0 else torch.float32, device="cuda")
+    g = torch.Generator(device="cuda")
+    g.manual_seed(7)
+    # orthonormal columns on every third row each, and a vector 0.05 away from their span
+    for c in range(k):
+        V[c, c:n:3] = torch.randn((n - c + 2) // 3, generator=g, dtype=V.dtype, device="cuda")
+        V[c] /= torch.linalg.vector_norm(V[c], dtype=torch.float64).to(V.dtype)
+    V[k, :n] = torch.randn(n, generator=g, dtype=V.dtype, device="cuda") * (0.05 / n ** 0.5)
+    for c in range(k):
+        V[k] += V[c] * (3.0, -2.0, 1.0)[c]
+    x, h = V[k].to(torch.float64, copy=True), torch.zeros(k, dtype=torch.float64)
+    for _ in range(2):
+        q = [float((V[c].double() * x).sum()) for c in range(k)]
+        onrm2 = float((x * x).sum())
+        for c in range(k):
+            x -= V[c].double() * q[c]
+        x = x.to(V.dtype).double()
+        h += torch.tensor(q, dtype=torch.float64)
+    nrm = (onrm2 - sum(a * a for a in q)) ** 0.5
+    torch.cuda.synchronize()
+    ctx = ks.Context()
+    buf = ks.DeviceArray.from_numpy(ctx, np.zeros((k + 2, 3), order="F"))
+    ctx.status_reset()
+    ks.check(ks.lib().ks_bv_orthonormalize_column_lean(ctx.h, prec, n, C.c_void_p(V.data_ptr()), ld, k, buf.ptr, k + 2, 2,
+                                                       2, 0, 0.7071, 1, 0), "orthonormalize")
+    st = ctx.status()
+    assert st.halt_col < 0 and st.lindep == 0 and st.error == 0 and st.total_passes == 2
+    hd = buf.numpy()[:, 2]
+    # dots of FP64 products, summed 64 rows in turn in 2,049 sub-chunks at most, then 2,048 workgroups: under
+    # 140,000 roundings in a row, 2e-11; the vector is 1/75 of w, its error as many times w's
+    assert np.abs(hd[:k] - h.numpy()).max() <= 2e-11 * 3.8
+    assert abs(hd[k] - nrm) <= 75 * 2e-11 * nrm and st.beta_last == hd[k]
+    x /= nrm
+    x -= V[k].double()
+    err = float(torch.linalg.vector_norm(x))
+    # FP32: the vector and the scaled vector are rounded once each
+    assert err <= 75 * 2e-11 + (0 if prec == 0 else 1.2e-7)
+    assert float(V[:, n].abs().max()) == 0
+    ctx.close()
+    del V, x
+    torch.cuda.empty_cache()
