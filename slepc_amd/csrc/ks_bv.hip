@@ -285,7 +285,7 @@ __device__ void gs_finish(const double *fin, int k, double *cbuf, double *hcol, 
 //   phase B  thread (column c, row class sub) accumulates column c . column k
 //            over rows sub, sub+T, ...  (c = k gives |w|^2), kept in registers
 //            across all sub-chunks of the workgroup.
-// A workgroup therefore reduces once, at the end, and the two-level finish
+// A workgroup therefore reduces once, at the end, and the separate finish
 // produces the k+1 dots.  FUSED=false is the first pass (c = V^T w, w^T w);
 // FUSED=true updates with this pass's c and returns the next pass's dots from
 // the updated vector, so a second DGKS pass costs one V read instead of two.
@@ -1601,7 +1601,7 @@ void launch_gs_fin(ks_ctx ctx, const gs_geom &g, int k, double *cbuf, double *hc
                        g.cw != 0 || g.kc != 0, halt_pass, coef1);
   else
     hipLaunchKernelGGL((k_gs_fin<FUSED>), dim3(k + 1), dim3(KS_FIN_BLOCK), 0, ctx->stream, ctx->d_partial, g.nb, k,
-                       ctx->d_gpartial, ctx->d_counters, cbuf, hcol, ctx->d_status, col, pass, refine, eta, do_scale,
+                       ctx->d_sums, ctx->d_counter, cbuf, hcol, ctx->d_status, col, pass, refine, eta, do_scale,
                        safe, deftol, g.cw != 0 || g.kc != 0, halt_pass, coef1);
   ks_prof_end(ctx);
 }
@@ -2003,10 +2003,10 @@ int ks_bv_orthonormalize_column_noalloc(void *stream, ks_prec prec, int n, void 
   ks_ctx_s c;
   c.stream = (hipStream_t)stream;
   c.d_status = (ks_status *)(base + KS_NOALLOC_STATUS);
-  c.d_counters = (unsigned *)(base + KS_NOALLOC_COUNTER);
-  c.d_gpartial = base + KS_NOALLOC_SUMS;
+  c.d_counter = (unsigned *)(base + KS_NOALLOC_COUNTER);
+  c.d_sums = base + KS_NOALLOC_SUMS;
   c.d_partial = base + KS_NOALLOC_PARTIAL;
-  hipLaunchKernelGGL(k_noalloc_reset, dim3(1), dim3(64), 0, c.stream, c.d_status, c.d_counters);
+  hipLaunchKernelGGL(k_noalloc_reset, dim3(1), dim3(64), 0, c.stream, c.d_status, c.d_counter);
   int err = prec == KS_F64 ? orthonormalize_t<double>(&c, n, (double *)V, ld, k, d_buf, ldbuf, hcol, col, refine,
                                                       eta, scale, safe)
                            : orthonormalize_t<float>(&c, n, (float *)V, ld, k, d_buf, ldbuf, hcol, col, refine,

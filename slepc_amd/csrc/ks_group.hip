@@ -101,9 +101,9 @@ int ks_group_step(ks_group g, int nmem, const ks_group_member *mem, ks_refine re
     G.cbuf = M.buf;                                        // buffer column 0: scratch coefficients
     G.hcol = M.buf + (size_t)M.hcol * (size_t)M.ldbuf;     // the column's h
     G.partial = M.ctx->d_partial;
-    G.sums = M.ctx->d_gpartial;
+    G.sums = M.ctx->d_sums;
     G.st = M.ctx->d_status;
-    G.counter = M.ctx->d_counters;
+    G.counter = M.ctx->d_counter;
     G.pub = M.ctx->d_finpub;
     G.coef1 = nullptr;   // grouped passes store every pass's vector (their sweep kernel takes no re-forming pass)
     G.ld = M.ld;

@@ -12,7 +12,6 @@
 #define KS_BLOCK 256                 // threads per block of the reduction kernels
 #define KS_WAVES (KS_BLOCK / 64)
 #define KS_MAXB 8192                 // maximum blocks of one row-partitioned reduction
-#define KS_GROUP 32                  // blocks per first-level reduction group
 #ifndef KS_GS_SPLITMAX
 #define KS_GS_SPLITMAX 128           // Gram-Schmidt against <= this many columns: column-split kernel
 #endif
@@ -51,7 +50,6 @@ __device__ __forceinline__ float2 ks_stream_load2(const float *p) {
 #ifndef KS_GS_BATCH
 #define KS_GS_BATCH 8                // column loads in flight per thread in the Gram-Schmidt sweep
 #endif
-#define KS_MAXG (KS_MAXB / KS_GROUP)
 #define KS_NCOLP (KS_MAX_COLS + 2)   // partial row width: columns + self dot + spare
 #ifndef KS_SPMV_NNZ
 #define KS_SPMV_NNZ 2048             // products staged in LDS per SpMV row block (a multiple of KS_BLOCK)
@@ -94,9 +92,9 @@ struct ks_ctx_s {
   hipStream_t stream = nullptr;
   ks_status *d_status = nullptr;
   double *d_partial = nullptr;     // [KS_MAXB][KS_NCOLP]
-  double *d_gpartial = nullptr;    // [KS_MAXG][KS_NCOLP]
-  unsigned *d_counters = nullptr;  // [KS_MAXG + 1], zero between launches
-  unsigned long long *d_finpub = nullptr;   // k_gs_fin's epoch and epoch-tagged sums [1 + 2 * KS_NCOLP]
+  double *d_sums = nullptr;        // k_gs_fin's column sums [KS_NCOLP] ...
+  unsigned *d_counter = nullptr;   // ... and its ticket, zero between launches
+  unsigned long long *d_finpub = nullptr;   // k_gs_fin_pub's epoch and epoch-tagged sums [1 + 2 * KS_NCOLP]
   double *d_coef1 = nullptr;                // first-pass coefficients kept for a deferred store [KS_NCOLP]
   double *d_scalar = nullptr;      // small device scratch (norm results)
   double *h_scalar = nullptr;      // pinned host scratch
