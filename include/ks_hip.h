@@ -149,7 +149,7 @@ int ks_csr_download(ks_csr A, ks_ctx ctx, int32_t *rowptr, int32_t *colidx, void
    B = diag(A - sigma I)^-1 from ks_pcg_jacobi (jacobi = 0: B = I).  Replaces
    STApply_Sinvert's KSPSolve (src/sys/classes/st/impls/sinvert/sinvert.c:16-30).
    The convergence tests run on the device; the host reads the solver state
-   once per 8 iterations.  d_work holds 4n + 64 doubles; reason > 0 converged,
+   once per 8 to 64 iterations (a quarter of those done).  d_work holds 4n + 64 doubles; reason > 0 converged,
    -3 iteration limit, -8 p^T (A - sigma I) p <= 0 (not positive definite). */
 int ks_pcg_jacobi(ks_ctx ctx, ks_csr A, double sigma, int jacobi, double *d_dinv);
 int ks_pcg_solve(ks_ctx ctx, ks_csr A, double sigma, const double *d_dinv, const double *d_b, double *d_x,
@@ -163,19 +163,19 @@ int ks_pcg_solve(ks_ctx ctx, ks_csr A, double sigma, const double *d_dinv, const
 int ks_bcgs_solve(ks_ctx ctx, ks_csr A, double sigma, const double *d_dinv, const double *d_b, double *d_x,
                   double rtol, double abstol, int maxits, double *d_work, int *its, double *rnorm, int *reason);
 /* QR of the n x k FP64 panel V (leading dimension ld) by TSQR: Householder QR
-   of row blocks of 2k rows (at least 64) in LDS, their triangular factors
+   of row blocks of 2k rows and more (a multiple of 64) in LDS, their triangular factors
    reduced by the same factorization up a tree.  R (k x k, host memory, leading
    dimension ldr) gets the factor; form_q != 0 overwrites V with Q, 0 leaves V
    as it is.  Replaces BVOrthogonalize_LAPACK_TSQR and _TSQR_OnlyR
    (src/sys/classes/bv/interface/bvlapack.c:347-560), which run LAPACK per
    process and reduce across processes.  Q and R are LAPACK's Householder QR up
-   to the signs of R's rows.  Allocates its workspace (about 1.5 n k doubles)
-   and waits for the stream. */
+   to the signs of R's rows.  Its workspace (about 1.5 n k doubles) is kept by the
+   context up to 256 MB, or taken from a current pool; waits for the stream. */
 int ks_bv_tsqr(ks_ctx ctx, int n, double *d_V, int ld, int k, int form_q, double *R, int ldr);
 /* ILU(0) of A - sigma I on A's pattern (Saad, Iterative Methods for Sparse Linear
    Systems, Algorithm 10.4; PETSc's PCILU with levels 0 and the natural
    ordering, its defaults), factored on the device one dependency level of rows
-   at a time; A's rows must list increasing columns and hold their diagonal.
+   after another, in a launch each or all in one; A's rows must list increasing columns and hold their diagonal.
    Fails with KS_ERR_PIVOT on a zero pivot.  Applying it is one launch for each
    factor: by levels in one workgroup where both factors have the layout that
    ks_ilu0_layout describes (and there is room for it), else rows pipelined through

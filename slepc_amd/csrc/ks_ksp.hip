@@ -19,8 +19,8 @@
 // previous one's per-workgroup partial sums (every workgroup adds the same
 // values in the same order) and takes the recurrence's scalars from them, and
 // the vector a product needs is formed on the fly where its entries are
-// gathered.  256 x 255 grid, one CG iteration: 22.3 us with a launch for each
-// operation and each sum, 12.8 us so (BiCGStab 40.9 and 19.0).
+// gathered.  256 x 255 grid, one CG iteration: 24.3 us with a launch for each
+// operation and each sum, 10.8 us so (BiCGStab 41.3 and 16.5).
 #include <algorithm>
 #include <cstring>
 #include <new>
@@ -581,7 +581,6 @@ __global__ __launch_bounds__(KS_ILU_WG) void k_ilu0_factor(const int32_t *__rest
   }
 }
 
-// one level of y = L^-1 y (unit lower factor), in place; skipped once the solve
 // One triangular solve of y = (L U)^-1 y in one launch (LOWER: the unit lower
 // factor, forward; else the upper factor, backward), in place, one wavefront per
 // row: row i goes to wavefront i (forward) or n-1-i (backward), so a row waits
@@ -780,9 +779,9 @@ inline ksp_run ksp_begin(ks_ctx ctx, ks_csr A, double *state, int nb) {
 // Products of up to this many entries form their vector as they gather it, one
 // launch fewer; beyond, the two or three gathers an entry cost more than the
 // launch.  us an iteration, formed inside / by itself: CG 256 x 255 grid (325,000
-// entries) 12.8 / 16.0, random graph of 900,000 entries 25.3 / 20.8, 512 x 511 grid
-// (1.3 million) 20.3 / 20.3; BiCGStab 19.0 / 26.6, 38.2 / 33.1, 32.5 / 35.1; CG on
-// 2048 x 2047 (21 million) 237 / 152.
+// entries) 10.8 / 12.2, random graph of 900,000 entries 24.6 / 18.5, 512 x 511 grid
+// (1.3 million) 19.5 / 18.3; BiCGStab 16.6 / 20.2, 40.5 / 29.9, 30.8 / 31.6; CG on
+// 2048 x 2047 (21 million) 186 / 154.
 #define KS_KSP_FUSE_NNZ 500000
 template <int MODE, bool PC>
 void ksp_product(ksp_run &R, ks_csr A, double sigma, const double *r, const double *p, const double *v,

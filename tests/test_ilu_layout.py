@@ -62,6 +62,7 @@ CASES = [  # matrix, rows of a step (0: none), threads, entries
     (lambda: layered([1500] * 7, 2), 1024, 1024, 2),      # two steps a level
     (lambda: layered([1500] * 7, 3), 512, 512, 4),        # three
     (lambda: layered([1000] + [3] * 1200, 2), 8, 64, 2),  # steps of 1024 would take 1,200 x 1024 slots
+    (lambda: layered([100] * 80, 2, far=True), 128, 128, 4),  # 10,240 slots back: the longest ring
     (lambda: layered([200] * 80, 2, far=True), 0, 0, 0),  # 20,480 slots back: past the ring
     (lambda: layered([50] * 40, 5), 0, 0, 0),             # more entries a row than it takes
     (lambda: layered([9000] * 2, 1), 0, 0, 0),            # nine steps a level: the whole chip's work
