@@ -659,12 +659,15 @@ __global__ __launch_bounds__(KS_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) v
 
 // The same sweep for more than KS_GS_SPLITMAX columns: eight wavefronts split
 // them, so CW (and the registers of a thread) stays at most 40.  FP32 data is
-// multiplied and summed in FP64, as the LDS-staged kernel does.  No pass defers
+// multiplied and summed in FP64, as the LDS-staged kernel does, a row a lane: two
+// (row pairs, as up to KS_GS_SPLITMAX columns) take 256 VGPRs and scratch at CW 40 (a
+// column, pairs / single rows: n = 405,224 k = 200 224 / 191 us, k = 319 763 / 337; n =
+// 4,000,000 k = 200 1743 / 1611, k = 319 6275 / 2648).  No pass defers
 // its store: the vector is less than a hundredth of what a sweep reads here, and
 // the re-forming sums cost as much or more (a column of n = 405,224: k = 130 245 us
 // against 256 with deferral, k = 200 385 and 391, k = 310 580 and 643).
 #define KS_GS_WIDE_WAVES 8
-template <typename T, int CW, bool FUSED, bool PAIR>
+template <typename T, int CW, bool FUSED>
 __global__ __launch_bounds__(64 * KS_GS_WIDE_WAVES) void k_gs_wide(const T *__restrict__ V, long ld, int k,
                                                                   T *__restrict__ w, int n, int rpb,
                                                                   const double *__restrict__ cbuf,
@@ -672,7 +675,7 @@ __global__ __launch_bounds__(64 * KS_GS_WIDE_WAVES) void k_gs_wide(const T *__re
                                                                   int col, int pass, int *ran) {
   if (!gs_pass_gate<FUSED>(st, col, pass)) return;
   if (ran && blockIdx.x == 0 && threadIdx.x == 0) *ran = 1;
-  gs_split_block<T, CW, FUSED, PAIR ? 2 : 1, PAIR, false, KS_GS_WIDE_WAVES, double>(
+  gs_split_block<T, CW, FUSED, 1, false, false, KS_GS_WIDE_WAVES, double>(
       blockIdx.x, gridDim.x, V, ld, k, w, n, rpb, cbuf, partial, gs_prescale<FUSED>(st, col, pass));
 }
 
@@ -1473,8 +1476,11 @@ int gs_geometry(int n, int k, size_t esize, gs_geom *g) {
   }
   // wider bases: the LDS-staged kernel only where a row's offset needs 64 bits.
   // A column (three sweeps), LDS-staged / split: n = 405,224 FP64 k = 130 329 / 245
-  // us, k = 200 627 / 385 (5.2-5.9 TB/s), k = 310 807 / 580; FP32 k = 200 1222 / 227;
-  // n = 5,000 k = 200 44 / 42.  1024 workgroups instead of 512: k = 200 416 us.
+  // us, k = 200 627 / 385 (5.2-5.9 TB/s), k = 310 807 / 580; FP32 k = 200 1208 / 191, k
+  // = 319 1382 / 337.  Short columns, a step of an expansion (which can leave out the
+  // scaling and a third pass only with the split): n = 2,025 FP64 k = 200 55 / 45, k =
+  // 305 57 / 54; FP32 59 / 45 and 59 / 54; by itself a column of n <= 4,000 with k > 220
+  // costs 2-6 us more (k = 319 47 / 53).  1024 workgroups instead of 512: k = 200 416 us.
   if ((uint64_t)n * esize < (1ull << 32)) {
     const int per = (k + KS_GS_WIDE_WAVES - 1) / KS_GS_WIDE_WAVES;
     static const int cws[] = {20, 24, 28, 32, 40};
@@ -1482,7 +1488,7 @@ int gs_geometry(int n, int k, size_t esize, gs_geom *g) {
     for (int c : cws)
       if (per <= c) { g->cw = c; break; }
     g->wide = 1;
-    const long step = esize == 4 ? 128 : 64;                            // rows per workgroup step, even
+    const long step = 64;                                               // rows per workgroup step
     const long tiles = (n + step - 1) / step;
     const long nb = tiles < KS_GS_WIDE_BLOCKS ? tiles : KS_GS_WIDE_BLOCKS;
     const long tpb = (tiles + nb - 1) / nb;
@@ -1544,12 +1550,8 @@ void launch_wide(ks_ctx ctx, const gs_geom &g, const T *V, long ld, int k, T *w,
   dim3 grid(g.nb), block(64 * KS_GS_WIDE_WAVES);
 #define KS_GSW_CASE(CC)                                                                                          \
   case CC:                                                                                                       \
-    if (g.pair)                                                                                                  \
-      hipLaunchKernelGGL((k_gs_wide<T, CC, FUSED, sizeof(T) == 4>), grid, block, 0, ctx->stream, V, ld, k, w, n, \
-                         g.cpb, cbuf, ctx->d_partial, ctx->d_status, col, pass, ran);                            \
-    else                                                                                                         \
-      hipLaunchKernelGGL((k_gs_wide<T, CC, FUSED, false>), grid, block, 0, ctx->stream, V, ld, k, w, n, g.cpb,   \
-                         cbuf, ctx->d_partial, ctx->d_status, col, pass, ran);                                   \
+    hipLaunchKernelGGL((k_gs_wide<T, CC, FUSED>), grid, block, 0, ctx->stream, V, ld, k, w, n, g.cpb, cbuf,      \
+                       ctx->d_partial, ctx->d_status, col, pass, ran);                                           \
     break;
   switch (g.cw) { KS_GSW_CASE(20) KS_GSW_CASE(24) KS_GSW_CASE(28) KS_GSW_CASE(32) KS_GSW_CASE(40) }
 #undef KS_GSW_CASE
@@ -1617,7 +1619,7 @@ int orthonormalize_t(ks_ctx ctx, int n, T *V, long ld, int k, double *buf, int l
   gs_geom g;
   int e;
   if ((e = gs_geometry(n, k, sizeof(T), &g))) return e;
-  g.pair = g.cw && sizeof(T) == 4 && ld % 2 == 0 && ((uintptr_t)V % 8) == 0;
+  g.pair = g.cw && !g.wide && sizeof(T) == 4 && ld % 2 == 0 && ((uintptr_t)V % 8) == 0;
   const double s = sizeof(T);
   T *w = V + (size_t)k * ld;
   double *cbuf = buf;                              // buffer column 0: scratch coefficients

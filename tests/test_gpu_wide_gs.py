@@ -17,7 +17,7 @@ KS = [128, 129, 160, 161, 192, 193, 224, 225, 256, 257, 319]
 def test_wide_orthonormalization(k, prec, pad):
     from slepc_amd import ks
     n = 2 * k + 64 * (k % 5) + 7
-    ld = (n + 1) // 2 * 2 + pad          # pad 1 with FP32: no row pairs
+    ld = (n + 1) // 2 * 2 + pad          # pad 1 with FP32: columns on 4-byte boundaries
     dt = np.float64 if prec == 0 else np.float32
     rng = np.random.default_rng(k)
     Q = np.linalg.qr(rng.standard_normal((n, k)))[0].astype(dt)
