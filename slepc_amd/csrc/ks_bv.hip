@@ -661,7 +661,7 @@ __global__ __launch_bounds__(KS_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) v
 // them, so CW (and the registers of a thread) stays at most 40.  FP32 data is
 // multiplied and summed in FP64, as the LDS-staged kernel does, a row a lane: two
 // (row pairs, as up to KS_GS_SPLITMAX columns) take 256 VGPRs and scratch at CW 40 (a
-// column, pairs / single rows: n = 405,224 k = 200 224 / 191 us, k = 319 763 / 337; n =
+// column, pairs / single rows: n = 405,224 k = 200 224 / 191 us, k = 319 763 / 329; n =
 // 4,000,000 k = 200 1743 / 1611, k = 319 6275 / 2648).  No pass defers
 // its store: the vector is less than a hundredth of what a sweep reads here, and
 // the re-forming sums cost as much or more (a column of n = 405,224: k = 130 245 us
@@ -1477,7 +1477,7 @@ int gs_geometry(int n, int k, size_t esize, gs_geom *g) {
   // wider bases: the LDS-staged kernel only where a row's offset needs 64 bits.
   // A column (three sweeps), LDS-staged / split: n = 405,224 FP64 k = 130 329 / 245
   // us, k = 200 627 / 385 (5.2-5.9 TB/s), k = 310 807 / 580; FP32 k = 200 1208 / 191, k
-  // = 319 1382 / 337.  Short columns, a step of an expansion (which can leave out the
+  // = 319 1382 / 329.  Short columns, a step of an expansion (which can leave out the
   // scaling and a third pass only with the split): n = 2,025 FP64 k = 200 55 / 45, k =
   // 305 57 / 54; FP32 59 / 45 and 59 / 54; by itself a column of n <= 4,000 with k > 220
   // costs 2-6 us more (k = 319 47 / 53).  1024 workgroups instead of 512: k = 200 416 us.

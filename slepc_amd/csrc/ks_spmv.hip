@@ -19,8 +19,9 @@ namespace {
 template <typename XT> struct acc_of { using type = double; };
 template <> struct acc_of<float> { using type = float; };
 
-// one row block b of y = A x (the body of both the single and the grouped kernel)
-template <typename VT, typename XT>
+// one row block b of y = A x (the body of both the single and the grouped kernel); LONG: the
+// matrix has rows of more than KS_SPMV_NNZ entries
+template <typename VT, typename XT, bool LONG>
 __device__ __forceinline__ void spmv_block(int b, const int32_t *__restrict__ blk, const int32_t *__restrict__ rowptr,
                                            const int32_t *__restrict__ colidx, const VT *__restrict__ val,
                                            const XT *__restrict__ x, XT *__restrict__ y) {
@@ -31,7 +32,7 @@ __device__ __forceinline__ void spmv_block(int b, const int32_t *__restrict__ bl
   const int r0 = blk[b], r1 = blk[b + 1];
   const int p0 = rowptr[r0], p1 = rowptr[r1];
   const int nrows = r1 - r0;
-  if (nrows == 1 && p1 - p0 > KS_SPMV_NNZ) {
+  if (LONG && nrows == 1 && p1 - p0 > KS_SPMV_NNZ) {
     // long row: the whole workgroup strides over it, PER entries a thread in flight: one
     // a time, the longest row (64,529 entries of an R-MAT graph of 2^20 vertices) took 252
     // round trips and the launch waited for it, 297 -> 211 us.  (Columns of the next step
@@ -97,7 +98,10 @@ __device__ __forceinline__ void spmv_block(int b, const int32_t *__restrict__ bl
   }
 }
 
-template <typename VT, typename XT>
+// Without long rows their code is left out: with it FP32 values and FP64 vectors take 65
+// VGPRs, seven wavefronts a SIMD, and a grid of 2048 x 2045 43.1 us instead of 40.2 (held to
+// eight wavefronts the R-MAT graph takes 215 us instead of 211)
+template <typename VT, typename XT, bool LONG>
 __global__ __launch_bounds__(KS_BLOCK) void k_spmv_csr(const int32_t *__restrict__ blk,
                                                        const int32_t *__restrict__ rowptr,
                                                        const int32_t *__restrict__ colidx,
@@ -106,7 +110,7 @@ __global__ __launch_bounds__(KS_BLOCK) void k_spmv_csr(const int32_t *__restrict
                                                        XT *__restrict__ y,
                                                        const ks_status *__restrict__ st) {
   if (st && !st->active) return;
-  spmv_block<VT, XT>(ks_xcd_block(blockIdx.x, gridDim.x), blk, rowptr, colidx, val, x, y);
+  spmv_block<VT, XT, LONG>(ks_xcd_block(blockIdx.x, gridDim.x), blk, rowptr, colidx, val, x, y);
 }
 
 // the SpMVs of several independent solves in one launch: workgroup b belongs to
@@ -115,7 +119,7 @@ __global__ __launch_bounds__(KS_BLOCK) void k_grp_spmv(ks_grp_spmv g) {
   int m = 0;
   while (m + 1 < g.nmem && (int)blockIdx.x >= g.b0[m + 1]) m++;
   if (!g.st[m]->active) return;
-  spmv_block<double, double>((int)blockIdx.x - g.b0[m], g.blk[m], g.rowptr[m], g.colidx[m], g.val[m], g.x[m],
+  spmv_block<double, double, true>((int)blockIdx.x - g.b0[m], g.blk[m], g.rowptr[m], g.colidx[m], g.val[m], g.x[m],
                              g.y[m]);
 }
 
@@ -306,18 +310,20 @@ int ks_spmv(ks_ctx ctx, ks_csr A, const void *x, void *y, ks_prec xprec, int gat
   const double bytes = (double)A->nnz * (vs + 4.0) + (A->nrows + 1.0) * 4.0 + A->ncols * xs + A->nrows * xs;
   ks_prof_begin(ctx, KS_PROF_SPMV, bytes, 2.0 * (double)A->nnz, false);
   dim3 grid(A->nblocks), block(KS_BLOCK);
-  if (A->vprec == KS_F64 && xprec == KS_F64)
-    hipLaunchKernelGGL((k_spmv_csr<double, double>), grid, block, 0, ctx->stream, A->d_blk, A->d_rowptr,
-                       A->d_colidx, (const double *)A->d_val, (const double *)x, (double *)y, st);
-  else if (A->vprec == KS_F32 && xprec == KS_F32)
-    hipLaunchKernelGGL((k_spmv_csr<float, float>), grid, block, 0, ctx->stream, A->d_blk, A->d_rowptr,
-                       A->d_colidx, (const float *)A->d_val, (const float *)x, (float *)y, st);
-  else if (A->vprec == KS_F32 && xprec == KS_F64)
-    hipLaunchKernelGGL((k_spmv_csr<float, double>), grid, block, 0, ctx->stream, A->d_blk, A->d_rowptr,
-                       A->d_colidx, (const float *)A->d_val, (const double *)x, (double *)y, st);
-  else
-    hipLaunchKernelGGL((k_spmv_csr<double, float>), grid, block, 0, ctx->stream, A->d_blk, A->d_rowptr,
-                       A->d_colidx, (const double *)A->d_val, (const float *)x, (float *)y, st);
+#define KS_SPMV_LAUNCH(VT, XT)                                                                                    \
+  do {                                                                                                            \
+    if (A->variant)                                                                                               \
+      hipLaunchKernelGGL((k_spmv_csr<VT, XT, true>), grid, block, 0, ctx->stream, A->d_blk, A->d_rowptr,          \
+                         A->d_colidx, (const VT *)A->d_val, (const XT *)x, (XT *)y, st);                          \
+    else                                                                                                          \
+      hipLaunchKernelGGL((k_spmv_csr<VT, XT, false>), grid, block, 0, ctx->stream, A->d_blk, A->d_rowptr,         \
+                         A->d_colidx, (const VT *)A->d_val, (const XT *)x, (XT *)y, st);                          \
+  } while (0)
+  if (A->vprec == KS_F64 && xprec == KS_F64) KS_SPMV_LAUNCH(double, double);
+  else if (A->vprec == KS_F32 && xprec == KS_F32) KS_SPMV_LAUNCH(float, float);
+  else if (A->vprec == KS_F32) KS_SPMV_LAUNCH(float, double);
+  else KS_SPMV_LAUNCH(double, float);
+#undef KS_SPMV_LAUNCH
   ks_prof_end(ctx);
   KS_HIP(hipGetLastError());
   return KS_OK;

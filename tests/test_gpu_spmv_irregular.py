@@ -7,7 +7,7 @@ pytestmark = pytest.mark.gpu
 
 ROWS = {"lengths": [2049, 2048, 2047, 0, 1, 4096, 4097, 6000, 16, 17, 33, 64, 65, 1000, 0],
         "short and long": ([3] * 200 + [40] + [900] + [2] * 50) * 3 + [5000],
-        "one": [9000], "few": [700, 600, 500, 2100, 1]}
+        "one": [9000], "few": [700, 600, 500, 2100, 1], "none long": [2048, 5, 0, 2047, 1, 2048] + [3] * 300}
 
 
 @pytest.mark.parametrize("vprec", [0, 1])
