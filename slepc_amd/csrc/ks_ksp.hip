@@ -957,7 +957,8 @@ int find_diagonals(int n, const int32_t *rp, const int32_t *ci, int32_t *diag) {
   for (int i = 0; i < n; i++) {
     diag[i] = -1;
     for (int32_t q = rp[i]; q < rp[i + 1]; q++) {
-      KS_CHECK(q == rp[i] || ci[q] > ci[q - 1], KS_ERR_ARG, "ILU(0) needs increasing column indices (row %d)", i);
+      KS_CHECK((q == rp[i] || ci[q] > ci[q - 1]) && ci[q] >= 0 && ci[q] < n, KS_ERR_ARG,
+               "ILU(0) needs increasing column indices (row %d)", i);
       if (ci[q] == i) diag[i] = q;
     }
     KS_CHECK(diag[i] >= 0, KS_ERR_ARG, "ILU(0) needs the diagonal entry of row %d", i);
@@ -1117,7 +1118,7 @@ int ks_ilu0_destroy(ks_ilu M) {
 }
 
 int ks_ilu0_layout(int n, const int32_t *rowptr, const int32_t *colidx, int lower, ks_ilu_layout *out) {
-  KS_CHECK(n > 0 && rowptr && colidx && out, KS_ERR_ARG, "bad ILU layout arguments");
+  KS_CHECK(n > 0 && rowptr && colidx && out && rowptr[0] == 0, KS_ERR_ARG, "bad ILU layout arguments");
   *out = ks_ilu_layout{};
   try {
     std::vector<int32_t> diag(n), rows, idx;

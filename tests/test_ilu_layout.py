@@ -92,3 +92,12 @@ def test_layout_memory_of_deep_levels(n):
     csr = M.laplacian_2d(n // 10, 10)
     for lower in (1, 0):
         assert 0 < layout(csr, lower).bytes <= 304 * n
+
+
+@pytest.mark.parametrize("rowptr,colidx", [([0, 1, 2], [1, 1]), ([0, 2, 3], [1, 0, 1]), ([0, 2, 3], [-1, 0, 1]),
+                                           ([0, 2, 3], [0, 2, 1]), ([0, 0, 1], [1]), ([1, 2, 3], [0, 0, 1])])
+def test_patterns_without_a_factorization_are_refused(rowptr, colidx):
+    # no diagonal, decreasing, negative, past the last column, an empty row, rows that start past 0
+    from slepc_amd import ks
+    with pytest.raises(ks.KSError):
+        layout((np.array(rowptr), np.array(colidx)), 1)
